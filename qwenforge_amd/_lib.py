@@ -1,5 +1,5 @@
 """ctypes binding of the C ABI in ``include/qf_attn.h``, ``include/qf_step.h``,
-``include/qf_paged.h`` and ``include/qf_probe.h``.
+``include/qf_wide.h``, ``include/qf_paged.h`` and ``include/qf_probe.h``.
 
 The shared object is built in-tree by ``qwenforge_amd.build``.  There is no
 fallback: if it is missing or does not load, every op raises.
@@ -221,6 +221,39 @@ SIGNATURES = {
         _vp, _i64, _vp,                 # w, w_sb, packed
         _i32, _i32, _i32,               # N, K, layout
         _vp,                            # stream
+    ],
+    # include/qf_wide.h
+    "qf_wide_qkv": [
+        _vp, _i64, _vp, _f32,           # x, x_sb, norm_w, eps
+        _vp, _vp, _vp, _vp,             # w_qkv, bias, pos, inv_freq
+        _vp, _i64, _i64, _i64,          # k_cache
+        _vp, _i64, _i64, _i64,          # v_cache
+        _vp, _i64, _i32, _i32, _i32,    # block_table, bt_sb, pages_per_row, n_pages, page_size
+        _vp, _i64,                      # slots, slot_sb
+        _vp, _i64, _i64,                # q_out, qo_sb, qo_sh
+        _i32, _i32, _i32, _i32, _i32, _i32,  # B, hidden, QH, KVH, D, cap
+        _vp,                            # stream
+    ],
+    "qf_wide_splits": [_i32],           # K
+    "qf_wide_gemv_residual": [
+        _vp, _i64, _vp, _vp, _i64,      # inp, in_sb, w, hidden, h_sb
+        _vp, _vp, _i32, _i32, _i32,     # part, ticket, B, K, N
+        _vp,                            # stream
+    ],
+    "qf_wide_gate_up": [
+        _vp, _i64, _vp, _f32, _vp,      # x, x_sb, norm_w, eps, w_gate_up
+        _vp, _i64, _i32, _i32, _i32,    # h_out, ho_sb, B, hidden, I
+        _vp,                            # stream
+    ],
+    "qf_wide_lm_head": [
+        _vp, _i64, _vp, _f32, _vp,      # x, x_sb, norm_w, eps, w_lm
+        _vp, _i64, _vp, _i32,           # logits, lg_sb, keys, n_blocks
+        _i32, _i32, _i32, _vp,          # B, hidden, V, stream
+    ],
+    "qf_wide_argmax_step": [
+        _vp, _i32, _i32, _vp,           # keys, n_blocks, B, token
+        _vp, _i64, _i32,                # rows, rows_sb, n_rows
+        _vp, _vp, _vp, _vp,             # step, write_index, pos, stream
     ],
     # include/qf_probe.h
     "qf_stream_read": [_vp, _i64, _vp, _i32, _vp],   # src, bytes, sink, workgroups, stream

@@ -23,7 +23,7 @@ LIB_PATH = PKG / "_qf_attn.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 SOURCES = ["decode_attn.hip", "decode_attn_fused_vec.hip", "prefill_attn.hip", "rope_append.hip",
-           "decode_step.hip", "probe.hip", "decode_valu.hip", "capi.cpp"]
+           "decode_step.hip", "decode_wide.hip", "probe.hip", "decode_valu.hip", "capi.cpp"]
 # Packed-fp32 VALU forms are disabled for all device code (they have produced
 # silently wrong results on this hardware pool); hipcc's host pass warns that it
 # does not know the feature, which is harmless.
@@ -42,6 +42,7 @@ COMMON_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", f"-I{ROO
 UNIT_FLAGS = {
     "decode_attn_fused_vec.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "decode_step.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
+    "decode_wide.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
 }
 
 

@@ -25,7 +25,7 @@
 // Replaces the torch op sequence of _decode_step_static
 // (student_engine.py:896-982); see include/qf_step.h for the per-entry-point
 // mapping and rounding.
-#include "qf_common.h"
+#include "step_common.h"
 #include "../../include/qf_step.h"
 #include "../../include/qf_paged.h"
 
@@ -34,12 +34,8 @@ namespace step {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kNW = 4;          // waves per workgroup
-constexpr int kNT = kNW * 64;   // threads per workgroup
 constexpr int kMaxB = 4;        // batch rows per launch
-constexpr int kMaxNormK = 1024; // widest normalised (hidden) row: one chunk per thread
 constexpr int kMaxK = 8192;     // widest projection input (down_proj: intermediate)
-constexpr int kHeadDim = 64;
 
 __device__ __forceinline__ float dot8(f16x8 w, f16x8 x, float acc) {
   acc = __builtin_amdgcn_fdot2(__builtin_shufflevector(w, w, 0, 1),
@@ -51,33 +47,6 @@ __device__ __forceinline__ float dot8(f16x8 w, f16x8 x, float acc) {
   acc = __builtin_amdgcn_fdot2(__builtin_shufflevector(w, w, 6, 7),
                                __builtin_shufflevector(x, x, 6, 7), acc, false);
   return acc;
-}
-
-// Sum over the 64 lanes with DPP moves (no LDS traffic): butterflies inside
-// each 16-lane row, then row broadcasts leave the total in lane 63, which is
-// read back as a wave-uniform value.
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ float dpp_add(float v) {
-  const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, kRowMask, 0xF,
-                                                false);
-  return v + __builtin_bit_cast(float, moved);
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-  v = dpp_add<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
-  v = dpp_add<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]: quad sums
-  v = dpp_add<0x141, 0xF>(v);  // row_half_mirror: 8-lane sums
-  v = dpp_add<0x140, 0xF>(v);  // row_mirror: 16-lane row sums
-  v = dpp_add<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
-  v = dpp_add<0x143, 0xC>(v);  // row_bcast:31 into rows 2, 3: lane 63 holds the total
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
-__device__ __forceinline__ f16x8 zero8() {
-  f16x8 z;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) z[e] = (f16)0.f;
-  return z;
 }
 
 // The NS 16-byte chunks of one weight row that lane `lane` multiplies:
@@ -191,20 +160,6 @@ __device__ __forceinline__ void plain_finish(const f16x8 (&v)[XP], int C, int NB
     if (idx < total) store16(xs + 8 * idx, v[i]);  // xs[b][c] at 8 * (b * C + c)
   }
   __syncthreads();
-}
-
-// Eager rotate-half RoPE of one (d, d+32) pair with the reference's fp16
-// rounding (student_engine.py:927-928): lo' = fp16(fp16(lo*cos_lo) -
-// fp16(hi*sin_lo)), hi' = fp16(fp16(hi*cos_hi) + fp16(lo*sin_hi)).
-__device__ __forceinline__ void rope1(float lo, float hi, float cl, float sl, float ch, float sh,
-                                      f16& out_lo, f16& out_hi) {
-#pragma clang fp contract(off)
-  const float a = round16(lo * cl);
-  const float b = round16(hi * sl);
-  const float c = round16(hi * ch);
-  const float d = round16(lo * sh);
-  out_lo = (f16)(a - b);
-  out_hi = (f16)(c + d);
 }
 
 // ---------------------------------------------------------------------------
@@ -705,11 +660,6 @@ __global__ __launch_bounds__(kNT) void rms_gate_up_swiglu_kernel(GateUpArgs a) {
 // k block kb) is the 1 KB A operand in lane order -- lane l's 16 bytes are
 // row r = l % 16, k = 32 kb + 8 (l / 16) .. +7 -- so every weight load of a
 // wave is one contiguous 1 KB read.  Tiles are stored rb-major.
-__device__ __forceinline__ f16x8 tile_load(const f16* __restrict__ w, int nkb, int rb, int kb,
-                                           int lane) {
-  return load16_nt(w + (((int64_t)rb * nkb + kb) * 64 + lane) * 8);
-}
-
 // B operand of k block kb for lane l: staged activation row l % 16 at
 // k = 32 kb + 8 (l / 16), zero for columns >= NB.
 template <int NB>
@@ -995,14 +945,6 @@ struct LmArgs {
   uint64_t* keys;
   int K, V;
 };
-
-// Orderable key of an fp16 logit at `index`: larger logit first, then the
-// smaller index (torch.argmax returns the first maximum).
-__device__ __forceinline__ uint64_t argmax_key(f16 v, int index) {
-  const unsigned short bits = __builtin_bit_cast(unsigned short, v);
-  const unsigned ord = (bits & 0x8000u) ? (~bits & 0xFFFFu) : (bits | 0x8000u);
-  return ((uint64_t)ord << 32) | (uint64_t)(0xFFFFFFFFu - (unsigned)index);
-}
 
 // Grid-stride over groups of RW rows per wave, next group's loads in flight
 // while the current one is reduced.

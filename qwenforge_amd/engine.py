@@ -28,8 +28,9 @@ path (``step_ops``, include/qf_step.h): per layer one launch for rms_norm +
 QKV + RoPE + append, the split-K attention launch, one for the split merge +
 o_proj + residual, one for rms_norm + gate/up + SwiGLU and one for down_proj +
 residual; then one for rms_norm + lm_head + per-block argmax and one for the
-argmax and the slot bookkeeping.  Larger batches keep the torch projections (hipBLASLt / ATen
-kernels) around the same HIP attention kernels.  Prefill always uses the torch
+argmax and the slot bookkeeping.  5..32 rows run the same step on the wide kernels
+(``wide_ops``, include/qf_wide.h) around the merged attention; larger batches keep the torch
+projections (hipBLASLt / ATen kernels) around the same HIP attention kernels.  Prefill always uses the torch
 projections.  Everything is fp16 storage with the reference's rounding points.
 """
 
@@ -40,7 +41,7 @@ from collections import OrderedDict
 import torch
 import torch.nn.functional as F
 
-from . import ops, step_ops
+from . import ops, step_ops, wide_ops
 from .model import Qwen2Config
 from .rope import cos_sin, inv_freq
 
@@ -117,6 +118,7 @@ class DecodeEngine:
         self._tiles = None
         self._lm_tiles = None
         self._o_tiles = None
+        self._down_tiles = None
         self._ctx = None
         self.graphs = GraphRegistry()
         self.captures = 0  # graph captures so far (registry hits capture nothing)
@@ -173,6 +175,39 @@ class DecodeEngine:
         """The fused decode-step kernels cover 1..4 rows and hidden <= 1024."""
         return (self.fused_step and 1 <= batch <= step_ops.MAX_BATCH and self.cfg.hidden <= 1024
                 and self.cfg.head_dim == step_ops.HEAD_DIM)
+
+    def down_weight_tiles(self, i: int):
+        """The packed down_proj weight of layer i for the wide step (packed
+        once, on first use)."""
+        if self._down_tiles is None:
+            self._down_tiles = [step_ops.pack_weight(l["down_weight"], step_ops.PACK_PLAIN)
+                                for l in self.w["layers"]]
+        return self._down_tiles[i]
+
+    def uses_wide_step(self, batch: int) -> bool:
+        """The wide decode-step kernels (``wide_ops``) cover 5..32 rows of the
+        shapes whose weights pack into tiles; other batches and shapes keep
+        the torch projections.  Measured on MI355X at Qwen2.5-0.5B shape and
+        1024 tokens of context, ms per step, torch projections / wide: B=5
+        1.69 / 0.71, B=8 1.73 / 0.73, B=12 1.71 / 0.78, B=16 1.69 / 0.82, B=32
+        1.97 / 1.07."""
+        cfg = self.cfg
+        if not (self.fused_step and self.tile_weights
+                and wide_ops.MIN_BATCH <= batch <= wide_ops.MAX_BATCH
+                and cfg.head_dim == step_ops.HEAD_DIM and cfg.hidden <= 1024
+                and cfg.hidden % 32 == 0 and cfg.intermediate % 32 == 0 and cfg.vocab % 16 == 0):
+            return False
+
+        def plain(t):
+            return (t.dtype == torch.float16 and t.device.type == "cuda" and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0)
+
+        norms = [l[k] for l in self.w["layers"] for k in ("input_norm", "post_norm")]
+        biases = [l["qkv_bias"] for l in self.w["layers"] if l["qkv_bias"] is not None]
+        mats = [l[k] for l in self.w["layers"]
+                for k in ("qkv_weight", "o_weight", "gate_up_weight", "down_weight")]
+        return all(plain(t) for t in (*norms, *biases, *mats, self.w["final_norm"],
+                                      self.w["lm_head"], self.w["embed"]))
 
     # ------------------------------------------------------------------ helpers
     def _rms(self, x, weight):
@@ -269,6 +304,8 @@ class DecodeEngine:
         """One static-shape decode step (the captured graph body)."""
         if ctx.get("fused"):
             self._step_fused(ctx)
+        elif ctx.get("wide"):
+            self._step_wide(ctx)
         else:
             self._step_torch(ctx)
 
@@ -312,6 +349,44 @@ class DecodeEngine:
                              ctx["keys"])
         step_ops.argmax_step(ctx["keys"], ctx["token"], ctx["rows"], ctx["step"], ctx["write"],
                              ctx["pos"])
+
+    def _step_wide(self, ctx):
+        """The step body on the wide kernels (5 <= B <= 32)."""
+        if ctx["bias"] is not None:
+            ctx["bias"].index_fill_(1, ctx["write"], 0.0)
+
+        def qkv(i, layer, w_qkv):
+            kc, vc = ctx["caches"][i]
+            wide_ops.rms_qkv_rope_append(ctx["hidden"], layer["input_norm"], self.cfg.rms_eps, w_qkv,
+                                         layer["qkv_bias"], (ctx["pos"], self.inv_freq), kc, vc,
+                                         ctx["write"], ctx["q_rot"])
+
+        def attend(i, grouped):
+            kc, vc = ctx["caches"][i]
+            return ops.flash_decode_attention(grouped, kc, vc, ctx["bias"], ctx["flash"],
+                                              kv_last=ctx["write"], scale=self.scale)
+
+        self._wide_body(ctx, qkv, attend, ctx["write"])
+
+    def _wide_body(self, ctx, qkv, attend, write):
+        """The wide step around one layer's ``qkv(i, layer, w_qkv)`` (norm, QKV,
+        RoPE and append into ``ctx["q_rot"]``) and ``attend(i, grouped)``."""
+        cfg = self.cfg
+        b = ctx["token"].shape[0]
+        hidden, h = ctx["hidden"], ctx["h"]
+        with torch.no_grad():  # out= takes no part in autograd, whatever the embedding does
+            torch.index_select(self.w["embed"], 0, ctx["token"], out=hidden)
+        grouped = ctx["q_rot"].view(b, cfg.kv_heads, cfg.groups, cfg.head_dim)
+        for i, layer in enumerate(self.w["layers"]):
+            w_qkv, w_gate_up = self.projection_weights(i, b)
+            qkv(i, layer, w_qkv)
+            att = attend(i, grouped).view(b, cfg.heads * cfg.head_dim)
+            wide_ops.gemv_residual(att, self.o_proj_weight(i, b), hidden, ctx["scratch"])
+            wide_ops.rms_gate_up_swiglu(hidden, layer["post_norm"], cfg.rms_eps, w_gate_up, h)
+            wide_ops.gemv_residual(h, self.down_weight_tiles(i), hidden, ctx["scratch"])
+        wide_ops.rms_lm_head(hidden, self.w["final_norm"], cfg.rms_eps, self.lm_head_weight(b),
+                             ctx["logits"], ctx["keys"])
+        wide_ops.argmax_step(ctx["keys"], ctx["token"], ctx["rows"], ctx["step"], write, ctx["pos"])
 
     def _step_torch(self, ctx):
         """The step body on torch projections around the HIP attention kernels."""
@@ -380,15 +455,24 @@ class DecodeEngine:
             "rows": torch.zeros(batch, max_new_tokens, device=dev, dtype=torch.long),
             "logits": torch.zeros(batch, cfg.vocab, device=dev, dtype=torch.float16),
             "fused": self.uses_fused_step(batch),
+            "wide": self.uses_wide_step(batch),
         }
-        if ctx["fused"]:
-            f16 = torch.float16
-            ctx["hidden"] = torch.zeros(batch, cfg.hidden, device=dev, dtype=f16)
-            ctx["q_rot"] = torch.zeros(batch, cfg.heads, cfg.head_dim, device=dev, dtype=f16)
-            ctx["h"] = torch.zeros(batch, cfg.intermediate, device=dev, dtype=f16)
-            ctx["keys"] = torch.zeros(batch, step_ops.lm_blocks(self.lm_head_weight(batch)),
-                                      device=dev, dtype=torch.long)
+        self._step_buffers(ctx, batch)
         return ctx
+
+    def _step_buffers(self, ctx, batch: int) -> None:
+        """The activations and scratch of a fused or wide step."""
+        if not (ctx["fused"] or ctx["wide"]):
+            return
+        cfg, dev, f16 = self.cfg, self.device, torch.float16
+        ctx["hidden"] = torch.zeros(batch, cfg.hidden, device=dev, dtype=f16)
+        ctx["q_rot"] = torch.zeros(batch, cfg.heads, cfg.head_dim, device=dev, dtype=f16)
+        ctx["h"] = torch.zeros(batch, cfg.intermediate, device=dev, dtype=f16)
+        ctx["keys"] = torch.zeros(batch, step_ops.lm_blocks(self.lm_head_weight(batch)),
+                                  device=dev, dtype=torch.long)
+        if ctx["wide"]:
+            ctx["scratch"] = wide_ops.make_wide_scratch(
+                batch, cfg.hidden, max(cfg.intermediate, cfg.heads * cfg.head_dim), dev)
 
     def capture(self, ctx):
         """Capture ``_step`` into a hipGraph (2 warm-ups on a side stream, SE:1056-1074).

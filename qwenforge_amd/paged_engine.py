@@ -16,8 +16,9 @@ pools (``paged.PagedKvCache``):
 
 The captured step is the dense engine's step with the paged kernels: for 1..4
 rows the fused weight-streaming kernels (QKV + RoPE + paged append, paged
-split-K attention, merge + o_proj, gate/up, down, lm_head + argmax), above
-that torch projections around the paged attention kernels.  Slots, positions,
+split-K attention, merge + o_proj, gate/up, down, lm_head + argmax), for 5..32
+rows their wide forms, above that torch projections around the paged attention
+kernels.  Slots, positions,
 tokens and the step counter advance on the device inside the graph.
 """
 
@@ -28,7 +29,7 @@ from collections import deque
 import torch
 import torch.nn.functional as F
 
-from . import ops, paged, step_ops
+from . import ops, paged, step_ops, wide_ops
 from .engine import DecodeEngine
 from .rope import cos_sin
 
@@ -88,14 +89,9 @@ class PagedDecodeEngine(DecodeEngine):
             "rows": torch.zeros(batch, n_cols, device=dev, dtype=torch.long),
             "logits": torch.zeros(batch, cfg.vocab, device=dev, dtype=torch.float16),
             "fused": fused,
+            "wide": self.uses_wide_step(batch),
         }
-        if fused:
-            f16 = torch.float16
-            ctx["hidden"] = torch.zeros(batch, cfg.hidden, device=dev, dtype=f16)
-            ctx["q_rot"] = torch.zeros(batch, cfg.heads, cfg.head_dim, device=dev, dtype=f16)
-            ctx["h"] = torch.zeros(batch, cfg.intermediate, device=dev, dtype=f16)
-            ctx["keys"] = torch.zeros(batch, step_ops.lm_blocks(self.lm_head_weight(batch)),
-                                      device=dev, dtype=torch.long)
+        self._step_buffers(ctx, batch)
         return ctx
 
     def _step(self, ctx):
@@ -103,6 +99,8 @@ class PagedDecodeEngine(DecodeEngine):
             return super()._step(ctx)
         if ctx["fused"]:
             self._step_fused_paged(ctx)
+        elif ctx["wide"]:
+            self._step_wide_paged(ctx)
         else:
             self._step_torch_paged(ctx)
 
@@ -134,6 +132,20 @@ class PagedDecodeEngine(DecodeEngine):
         step_ops.rms_lm_head(hidden, self.w["final_norm"], eps, self.lm_head_weight(b), ctx["logits"],
                              ctx["keys"])
         step_ops.argmax_step(ctx["keys"], ctx["token"], ctx["rows"], ctx["step"], None, pos)
+
+    def _step_wide_paged(self, ctx):
+        kv, table, pos = ctx["kv"], ctx["table"], ctx["pos"]
+
+        def qkv(i, layer, w_qkv):
+            wide_ops.rms_qkv_rope_append_paged(ctx["hidden"], layer["input_norm"], self.cfg.rms_eps,
+                                               w_qkv, layer["qkv_bias"], (pos, self.inv_freq),
+                                               *kv.pools[i], table, pos, ctx["q_rot"])
+
+        def attend(i, grouped):
+            return paged.flash_decode_attention_paged(grouped, *kv.pools[i], table, None,
+                                                      ctx["flash"], kv_last=pos, scale=self.scale)
+
+        self._wide_body(ctx, qkv, attend, None)
 
     def _step_torch_paged(self, ctx):
         cfg = self.cfg

@@ -1,0 +1,183 @@
+"""Decode-step kernels for 5..32 rows (include/qf_wide.h) against ``oracle.step``.
+
+Batches sit at the edges of the kernels' tiles: the fewest rows, whole and
+ragged blocks of four rows (rows per wave) and of 16 (matrix-core columns),
+the most rows.  Integer operands make every sum exact in any order, so those
+outputs match bit for bit; random ones agree to a few fp16 ulps (the bound of
+the 1..4-row kernels' tests).
+"""
+
+import pytest
+import torch
+
+import oracle.step as ost
+from oracle.rope import inv_freq, rope_cos_sin
+from qwenforge_amd import step_ops, wide_ops
+from qwenforge_amd.engine import DecodeEngine
+from qwenforge_amd.model import Qwen2Config, init_weights
+from qwenforge_amd.paged_engine import PagedDecodeEngine
+
+pytestmark = pytest.mark.gpu
+
+HIDDEN, QH, KVH, D, INTER = 896, 14, 2, 64, 4864
+EPS = 1e-6
+STEP_TOL = 4e-3   # |got - ref| <= STEP_TOL * max(1, |ref|)
+LOGIT_TOL = 3e-2  # the engine tests' bound
+BATCHES = [5, 8, 13, 16, 17, 32]
+
+
+def _close(got, ref):
+    return (((got.float().cpu() - ref.float()).abs()) / ref.float().abs().clamp_min(1.0)).max().item()
+
+
+def _int_rows(b, n, gen):
+    return (torch.randint(0, 2, (b, n), generator=gen) * 2 - 1).half()
+
+
+def _int_w(n, k, gen):
+    return torch.randint(-1, 2, (n, k), generator=gen).half()
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("hidden", [HIDDEN, 96, 1024])
+def test_qkv_rope_append_exact(dev, batch, hidden, paged):
+    gen = torch.Generator().manual_seed(batch + hidden)
+    x, nw = _int_rows(batch, hidden, gen), torch.ones(hidden, dtype=torch.float16)
+    width = (QH + 2 * KVH) * D
+    w, bias = _int_w(width, hidden, gen), torch.randint(-3, 4, (width,), generator=gen).half()
+    pos = torch.randint(0, 40000, (batch,), generator=gen)
+    cos, sin = rope_cos_sin(pos, inv_freq(D, 1e6))
+    q, k, v = ost.qkv_rope16(x, nw, EPS, w, bias, cos, sin, QH, KVH, D)
+    tiles = step_ops.pack_weight(w.to(dev), step_ops.PACK_ROPE)
+    q_out = torch.zeros(batch, QH, D, device=dev, dtype=torch.float16)
+    positions = (pos.to(dev), inv_freq(D, 1e6).to(dev))
+    print(f"[wide qkv] B={batch} hidden={hidden} paged={paged}", flush=True)
+    if paged:
+        # One row's slot is past its pages and one page is unmapped: nothing is written there.
+        kc = torch.zeros(2 * batch, KVH, 64, D, device=dev, dtype=torch.float16)
+        vc = torch.zeros_like(kc)
+        table = torch.randperm(2 * batch, generator=gen).to(torch.int32).view(batch, 2)
+        slots = torch.randint(0, 128, (batch,), generator=gen)
+        slots[0], slots[1] = 128, 5
+        table[1, 0] = -1
+        wide_ops.rms_qkv_rope_append_paged(x.to(dev), nw.to(dev), EPS, tiles, bias.to(dev), positions,
+                                           kc, vc, table.to(dev), slots.to(dev), q_out)
+        kr, vr = torch.zeros_like(kc, device="cpu"), torch.zeros_like(kc, device="cpu")
+        for b in range(2, batch):
+            page = int(table[b, int(slots[b]) // 64])
+            kr[page, :, int(slots[b]) % 64], vr[page, :, int(slots[b]) % 64] = k[b], v[b]
+    else:
+        kc = torch.zeros(batch, KVH, 64, D, device=dev, dtype=torch.float16)
+        vc = torch.zeros_like(kc)
+        wide_ops.rms_qkv_rope_append(x.to(dev), nw.to(dev), EPS, tiles, bias.to(dev), positions,
+                                     kc, vc, torch.tensor([37], device=dev), q_out)
+        kr, vr = torch.zeros_like(kc, device="cpu"), torch.zeros_like(kc, device="cpu")
+        kr[:, :, 37], vr[:, :, 37] = k, v
+    assert torch.equal(q_out.cpu(), q)
+    assert torch.equal(kc.cpu(), kr) and torch.equal(vc.cpu(), vr)
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("k_dim,n", [(HIDDEN, HIDDEN), (INTER, HIDDEN), (32, 16), (1024, 48),
+                                     (1056, 32), (8192, 64)])
+def test_gemv_residual_exact_on_repeated_calls(dev, batch, k_dim, n):
+    gen = torch.Generator().manual_seed(batch + k_dim)
+    w = _int_w(n, k_dim, gen)
+    tiles = step_ops.pack_weight(w.to(dev), step_ops.PACK_PLAIN)
+    scratch = wide_ops.make_wide_scratch(batch, n, k_dim, dev)
+    print(f"[wide gemv] B={batch} K={k_dim} N={n}", flush=True)
+    for _ in range(3):  # the ticket re-arms
+        inp = _int_rows(batch, k_dim, gen)
+        res = torch.randint(-8, 9, (batch, n), generator=gen).half()
+        hidden = res.to(dev)
+        wide_ops.gemv_residual(inp.to(dev), tiles, hidden, scratch)
+        assert torch.equal(hidden.cpu(), ost.residual16(res, inp, w))
+    assert not bool(scratch[1].any())
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("hidden,inter", [(HIDDEN, INTER), (64, 40)])
+def test_gate_up_swiglu(dev, batch, hidden, inter):
+    gen = torch.Generator().manual_seed(batch)
+    x = torch.randn(batch, hidden, generator=gen).half()
+    nw = (torch.rand(hidden, generator=gen) + 0.5).half()
+    w = (torch.randn(2 * inter, hidden, generator=gen) * 0.02).half()
+    h = torch.zeros(batch, inter, device=dev, dtype=torch.float16)
+    print(f"[wide gate_up] B={batch} {hidden}x{inter}", flush=True)
+    wide_ops.rms_gate_up_swiglu(x.to(dev), nw.to(dev), EPS,
+                                step_ops.pack_weight(w.to(dev), step_ops.PACK_SWIGLU), h)
+    assert _close(h, ost.swiglu16(x, nw, EPS, w)) <= STEP_TOL
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("blocks", [1, 96, 512])
+def test_lm_head_and_argmax_step_exact(dev, batch, blocks):
+    """Integer logits, a planted tie (first index wins) and a row of NaNs
+    (torch.argmax names the first)."""
+    gen = torch.Generator().manual_seed(batch)
+    vocab = 5008
+    x, nw = _int_rows(batch, HIDDEN, gen), torch.ones(HIDDEN, dtype=torch.float16)
+    w = _int_w(vocab, HIDDEN, gen)
+    w[1234] = torch.sign(x[0].float()).half()
+    w[4000] = w[1234]
+    x[1, 5] = float("nan")
+    logits = torch.zeros(batch, vocab, device=dev, dtype=torch.float16)
+    keys = torch.zeros(batch, blocks, device=dev, dtype=torch.long)
+    print(f"[wide lm_head] B={batch} blocks={blocks}", flush=True)
+    wide_ops.rms_lm_head(x.to(dev), nw.to(dev), EPS, step_ops.pack_weight(w.to(dev)), logits, keys)
+    token, rows = torch.full((batch,), -1, device=dev), torch.zeros(batch, 5, device=dev).long()
+    step, write = torch.tensor([2], device=dev), torch.tensor([40], device=dev)
+    pos = torch.arange(batch, device=dev) + 10
+    wide_ops.argmax_step(keys, token, rows, step, write, pos)
+    ref, first = ost.lm_head_argmax(x, nw, EPS, w)
+    keep = [b for b in range(batch) if b != 1]
+    assert torch.equal(logits.cpu()[keep], ref[keep]) and bool(logits[1].isnan().all())
+    first[1] = 0
+    assert int(first[0]) == 1234 and torch.equal(token.cpu(), first)
+    assert torch.equal(rows.cpu()[:, 2], first) and not bool(rows[:, [0, 1, 3, 4]].any())
+    assert int(step) == 3 and int(write) == 41 and torch.equal(pos.cpu(), torch.arange(batch) + 11)
+
+
+@pytest.mark.parametrize("batch,paged", [(5, False), (16, True), (17, False), (32, True)])
+def test_wide_step_matches_torch_step(dev, batch, paged):
+    """Teacher-forced logits, appended rows and bookkeeping of the captured
+    wide step equal the torch-projection step's within the engine's bound."""
+    cfg = Qwen2Config(layers=3)
+    w = init_weights(cfg, dev, seed=3)
+    s, steps = 70, 3
+    gen = torch.Generator().manual_seed(5)
+    ids = torch.randint(0, cfg.vocab, (batch, s), generator=gen).to(dev)
+    teacher = torch.randint(0, cfg.vocab, (steps, batch), generator=gen).to(dev)
+    out = {}
+    for wide in (True, False):
+        eng = (PagedDecodeEngine if paged else DecodeEngine)(cfg, w, dev, tile_weights=wide)
+        if paged:
+            kv = eng.new_paged_cache(batch, 2 * batch, 64, 2)
+            for r in range(batch):
+                kv.map_row(r, 128)
+            eng.prefill_paged(list(ids), kv, range(batch))
+            ctx = eng.make_paged_context(kv, batch, steps + 1)
+            eng.capture_paged(ctx)
+        else:
+            caches = eng.new_caches(batch, 128)
+            eng.prefill(ids, caches)
+            ctx = eng.make_context(caches, batch, steps + 1)
+            eng.capture(ctx)
+            ctx["write"].fill_(s)
+        assert ctx["wide"] == wide
+        ctx["pos"].fill_(s)
+        ctx["step"].fill_(1)
+        logits = []
+        for t in range(steps):
+            ctx["token"].copy_(teacher[t])
+            ctx["graph"].replay()
+            logits.append(ctx["logits"].float().cpu())
+        rows = ([kv.gather(i, r, s + steps)[0] for i in range(3) for r in range(batch)] if paged
+                else [k[:, :, s:s + steps] for k, _ in caches])
+        out[wide] = (torch.stack(logits), ctx["pos"].cpu(), int(ctx["step"]),
+                     torch.stack([r.float().cpu() for r in rows]))
+    (lw, pw, sw, cw), (lt, pt, st, ct) = out[True], out[False]
+    print(f"[wide vs torch step B={batch}] max|dlogit| {(lw - lt).abs().max():.3e}", flush=True)
+    assert (lw - lt).abs().max().item() <= LOGIT_TOL
+    assert torch.equal(pw, pt) and sw == st and (cw - ct).abs().max().item() <= 2e-2
