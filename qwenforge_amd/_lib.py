@@ -1,5 +1,5 @@
 """ctypes binding of the C ABI in ``include/qf_attn.h``, ``include/qf_step.h``,
-``include/qf_wide.h``, ``include/qf_paged.h`` and ``include/qf_probe.h``.
+``include/qf_wide.h``, ``include/qf_prefill.h``, ``include/qf_paged.h`` and ``include/qf_probe.h``.
 
 The shared object is built in-tree by ``qwenforge_amd.build``.  There is no
 fallback: if it is missing or does not load, every op raises.
@@ -255,6 +255,16 @@ SIGNATURES = {
         _vp, _i64, _i32,                # rows, rows_sb, n_rows
         _vp, _vp, _vp, _vp,             # step, write_index, pos, stream
     ],
+    # include/qf_prefill.h
+    "qf_prefill_layers_workspace": [_i32, _i32, _i32, _i32, _i32, _i32],  # T, hidden, QH, KVH, D, I
+    "qf_prefill_layers": [
+        _vp, _i32, _vp, _i32, _i32, _i32,  # layers, n_layers, hidden, T, B, S
+        _vp, _vp,                       # cu, inv_freq
+        _vp, _i64, _i32, _i32, _i32,    # block_table, bt_sb, pages_per_row, n_pages, page_size
+        _vp, _i64, _f32,                # ws, ws_bytes, eps
+        _i32, _i32, _i32, _i32, _i32,   # hidden_size, QH, KVH, D, I
+        _vp,                            # stream
+    ],
     # include/qf_probe.h
     "qf_stream_read": [_vp, _i64, _vp, _i32, _vp],   # src, bytes, sink, workgroups, stream
     "qf_launch_probe": [_vp, _i64, _vp, _vp,          # src, bytes, index, sink
@@ -273,7 +283,7 @@ SIGNATURES = {
 }
 
 # Entry points that do not return an int status.
-RESTYPES = {"qf_error_string": C.c_char_p}
+RESTYPES = {"qf_error_string": C.c_char_p, "qf_prefill_layers_workspace": _i64}
 
 _lock = threading.Lock()
 _lib: C.CDLL | None = None

@@ -909,7 +909,7 @@ using qf::prefill::Args;
 // Shared launch sequence of the dense and the packed (varlen) entry points;
 // `a` is filled and validated.  Returns 0 or a QF_ERR_* / hipError_t code.
 // CUs of the device that owns `st` (cached per device); 0 if it cannot be read.
-static int stream_cus(hipStream_t st) {
+int qf::stream_cus(hipStream_t st) {
   constexpr int kMaxDevices = 64;
   static std::atomic<int> cached[kMaxDevices];
   int dev = -1;
@@ -979,7 +979,7 @@ static int prefill_launch(Args a, bool rope, bool append, hipStream_t st) {
   // the unpaired heaviest tiles take about 0.1 us more off the attention.
   a.snake = 0;
   {
-    const int cus = stream_cus(st);
+    const int cus = qf::stream_cus(st);
     if (cus > 0 && lgrid.x > (unsigned)cus && lgrid.x <= 2u * (unsigned)cus) a.snake = cus;
   }
   if (paged) {

@@ -184,6 +184,9 @@ __device__ __forceinline__ float col_sum(float x) {
   return a + b;
 }
 
+// Compute units of the device of `st` (prefill_attn.hip), 0 if unknown.
+int stream_cus(hipStream_t st);
+
 // Paged KV caches (host side): page_size must be a power of two in
 // [64, 4096] (a 32-key decode tile and a 64-key prefill tile then never
 // straddle a page), with at least one page per row and a non-empty pool.

@@ -41,7 +41,7 @@ from collections import OrderedDict
 import torch
 import torch.nn.functional as F
 
-from . import ops, step_ops, wide_ops
+from . import ops, prefill_ops, step_ops, wide_ops
 from .model import Qwen2Config
 from .rope import cos_sin, inv_freq
 
@@ -243,6 +243,8 @@ class DecodeEngine:
         cfg = self.cfg
         b, s = input_ids.shape
         hidden = F.embedding(input_ids, self.w["embed"])
+        if self._native_layers(hidden, caches, (b, cfg.kv_heads, s, cfg.head_dim), b, s):
+            return self._last_logits(hidden[:, -1])
         cos, sin = cos_sin(torch.arange(s, device=self.device), self.inv_freq)
         for layer, (kc, vc) in zip(self.w["layers"], caches):
             residual = hidden
@@ -252,8 +254,25 @@ class DecodeEngine:
             hidden = residual + F.linear(att, layer["o_weight"])
             residual = hidden
             hidden = residual + self._mlp(self._rms(hidden, layer["post_norm"]), layer)
-        last = self._rms(hidden[:, -1], self.w["final_norm"])
-        return F.linear(last, self.w["lm_head"])
+        return self._last_logits(hidden[:, -1])
+
+    def _last_logits(self, last):
+        return F.linear(self._rms(last, self.w["final_norm"]), self.w["lm_head"])
+
+    def _native_layers(self, hidden, caches, shape, rows: int, longest: int, **paged) -> bool:
+        """Runs every layer over ``hidden`` in place with one native call
+        (``prefill_ops``), or returns False where the model's or the caches'
+        layout is one it does not take (the torch projections then run)."""
+        cfg = self.cfg
+        tokens = hidden.numel() // cfg.hidden
+        if (tokens < 1 or longest < 1 or hidden.dtype != torch.float16 or not hidden.is_cuda
+                or prefill_ops.workspace_bytes(cfg, tokens) < 0):
+            return False
+        table = prefill_ops.layer_table(cfg, self.w["layers"], caches, hidden.device, shape)
+        if table is None:
+            return False
+        prefill_ops.prefill_layers(cfg, table, hidden, rows, longest, self.inv_freq, **paged)
+        return True
 
     @torch.no_grad()
     def prefill_ragged(self, prompts, caches):
@@ -266,12 +285,16 @@ class DecodeEngine:
         """
         return self._prefill_packed(
             prompts, lambda i, q, k, v, cu, n, cos, sin, lengths: ops.prefill_varlen(
-                q, k, v, cu, n, cos, sin, caches[i][0], caches[i][1], 0, lengths=lengths))
+                q, k, v, cu, n, cos, sin, caches[i][0], caches[i][1], 0, lengths=lengths),
+            lambda hidden, cu, longest: self._native_layers(
+                hidden, caches, (len(prompts), self.cfg.kv_heads, longest, self.cfg.head_dim),
+                len(prompts), longest, cu=cu))
 
-    def _prefill_packed(self, prompts, attend):
-        """Packed ragged prefill body; ``attend(layer, q, k, v, cu, max_len, cos,
-        sin, lengths)`` runs the varlen RoPE + append + attention launch of one
-        layer (``lengths``: the host row lengths ``cu`` was built from)."""
+    def _prefill_packed(self, prompts, attend, native):
+        """Packed ragged prefill body; ``native(hidden, cu, max_len)`` runs all
+        layers in one call if it can; else ``attend(layer, q, k, v, cu, max_len,
+        cos, sin, lengths)`` runs the varlen RoPE + append + attention launch of
+        one layer (``lengths``: the host row lengths ``cu`` was built from)."""
         cfg = self.cfg
         dev = self.device
         lengths = [int(p.numel()) for p in prompts]
@@ -281,10 +304,12 @@ class DecodeEngine:
         for n in lengths:
             starts.append(starts[-1] + n)
         cu = torch.tensor(starts, dtype=torch.int32, device=dev)
+        hidden = F.embedding(ids, self.w["embed"])
+        if native(hidden, cu, max(lengths)):
+            return self._last_logits(hidden[cu[1:].long() - 1])
         pos = torch.cat([torch.arange(n, device=dev) for n in lengths])
         cos, sin = cos_sin(pos, self.inv_freq)                 # (T, D): each row's own positions
         qw, kvw = cfg.heads * cfg.head_dim, cfg.kv_heads * cfg.head_dim
-        hidden = F.embedding(ids, self.w["embed"])
         for i, layer in enumerate(self.w["layers"]):
             residual = hidden
             proj = F.linear(self._rms(hidden, layer["input_norm"]), layer["qkv_weight"],
@@ -296,8 +321,7 @@ class DecodeEngine:
             hidden = residual + F.linear(att.reshape(total, cfg.hidden), layer["o_weight"])
             residual = hidden
             hidden = residual + self._mlp(self._rms(hidden, layer["post_norm"]), layer)
-        last = hidden[cu[1:].long() - 1]
-        return F.linear(self._rms(last, self.w["final_norm"]), self.w["lm_head"])
+        return self._last_logits(hidden[cu[1:].long() - 1])
 
     # ------------------------------------------------------------------ decode
     def _step(self, ctx):

@@ -61,7 +61,11 @@ class PagedDecodeEngine(DecodeEngine):
         return self._prefill_packed(
             prompts, lambda i, q, k, v, cu, n, cos, sin, lengths: paged.prefill_varlen_paged(
                 q, k, v, cu, n, cos, sin, kv.pools[i][0], kv.pools[i][1], table, 0,
-                lengths=lengths))
+                lengths=lengths),
+            lambda hidden, cu, longest: longest <= kv.capacity and self._native_layers(
+                hidden, kv.pools, (kv.n_pages, kv.kv_heads, kv.page_size, self.cfg.head_dim),
+                len(prompts), longest, cu=cu, block_table=table, n_pages=kv.n_pages,
+                page_size=kv.page_size))
 
     # ------------------------------------------------------------------ decode
     def make_paged_context(self, kv: paged.PagedKvCache, batch: int, n_cols: int):
