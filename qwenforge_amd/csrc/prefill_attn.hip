@@ -34,6 +34,7 @@
 // rescaled when the running max grows by more than kRescaleSlack); Q is
 // rotated in registers once at the start.  The causal mask is applied only on
 // the diagonal and tail tiles.
+#include <algorithm>
 #include <atomic>
 
 #include "qf_common.h"
@@ -659,8 +660,8 @@ __device__ __forceinline__ void tile_compute(LdsCtx& c, int kt, const unsigned c
 // step i + 1 are issued after step i's barrier, when every wave is done with
 // step i - 1's stage.  At the end groups 1 .. kG-1 hand their softmax states
 // to group 0 through LDS, which merges them.  The heaviest query tile takes
-// 1/kG of the steps, with no partial or merge through memory.  kG = 2: two
-// workgroups per CU; kG = 4: one (both four waves per SIMD).
+// 1/kG of the steps, with no partial or merge through memory.  Four waves per
+// SIMD: kG = 2 two workgroups per CU, kG = 1 four.
 constexpr int kTileBytes = kBN * kRowBytes;
 
 template <int kG, bool kRopeQ, bool kPaged>
@@ -931,6 +932,21 @@ int qf::stream_cus(hipStream_t st) {
   return cus;
 }
 
+// The streaming kernel with kG wave groups per query tile.
+template <int kG>
+static int launch_stream(const Args& a, bool rope, bool paged, dim3 grid, hipStream_t st) {
+  using namespace qf::prefill;
+  const dim3 block(kG * 4 * 64);
+  if (paged) {
+    if (rope) hipLaunchKernelGGL((prefill_lds2_kernel<kG, true, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_lds2_kernel<kG, false, true>), grid, block, 0, st, a);
+  } else {
+    if (rope) hipLaunchKernelGGL((prefill_lds2_kernel<kG, true, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((prefill_lds2_kernel<kG, false, false>), grid, block, 0, st, a);
+  }
+  return (int)hipGetLastError();
+}
+
 static int prefill_launch(Args a, bool rope, bool append, hipStream_t st) {
   using namespace qf::prefill;
   const int B = a.B, QH = a.QH, KVH = a.KVH, S = a.S;
@@ -965,10 +981,26 @@ static int prefill_launch(Args a, bool rope, bool append, hipStream_t st) {
   // One eight-wave workgroup per (query tile, b * QH + q head).
   if ((int64_t)grid.x * B * QH > 0x7fffffff) return QF_ERR_UNSUPPORTED;
   const dim3 lgrid((unsigned)(grid.x * B * QH));
-  // Two groups (measured on MI355X: four, one 16-wave workgroup per CU,
-  // were slower at every size, 28.8 vs 26.0 us at S=2048).
-  constexpr int G = 2;
-  const dim3 lblock(G * 4 * 64);
+  // Two wave groups per query tile (four, one 16-wave workgroup per CU, were
+  // slower at every size, 28.8 vs 26.0 us at S=2048), or one.  One group
+  // doubles the steps of the heaviest tile, but then four independent
+  // workgroups share a CU instead of two whose groups keep in step, and no
+  // states are merged: faster once the tiles fill the CUs more than once (two
+  // per CU) and no chain stands out -- at least 24 tiles for each step of the
+  // longest (batches), or five tiles per CU.  Measured on MI355X, us per call
+  // for 14 heads, two groups / one: B=8 S=300 15.4 / 13.6, S=500 20.1 / 17.9,
+  // S=1000 39.4 / 34.8, B=4 S=700 18.9 / 17.4, S=2048 57.4 / 52.6, B=2 S=2048
+  // 35.1 / 34.0, 16 packed rows of 25-500 21.7 / 18.3, B=1 S=6000 100.7 / 95.3;
+  // outside the rule B=4 S=500 13.3 / 14.2, B=1 S=2048 23.4 / 29.0, S=3072 35.2
+  // / 41.0, S=4096 55.9 / 56.8.
+  const int cus = stream_cus(st);
+  // Packed rows: at most total / 64 + B tiles (equal rows count as dense ones).
+  int64_t tiles = (int64_t)lgrid.x;
+  if (a.cu != nullptr) tiles = std::min(tiles, (int64_t)(a.total / kBM + B) * QH);
+  if (cus > 0 && tiles > 2 * cus && (tiles >= 24 * (int64_t)grid.x || tiles >= 5 * cus)) {
+    a.snake = 0;
+    return launch_stream<1>(a, rope, paged, lgrid, st);
+  }
   // Two workgroups fit a CU.  When the grid needs more than one per CU but
   // no more than two, the first round (one per CU) shares most CUs with a
   // second-round workgroup.  The heaviest query tiles go to the CUs that get
@@ -977,19 +1009,8 @@ static int prefill_launch(Args a, bool rope, bool append, hipStream_t st) {
   // MI355X, same outputs, against heaviest-first throughout: S=2048 call 23.4
   // -> 22.9 us, S=1536 18.8 -> 18.6, S=2304 26.1 -> 25.45 with the pairing;
   // the unpaired heaviest tiles take about 0.1 us more off the attention.
-  a.snake = 0;
-  {
-    const int cus = qf::stream_cus(st);
-    if (cus > 0 && lgrid.x > (unsigned)cus && lgrid.x <= 2u * (unsigned)cus) a.snake = cus;
-  }
-  if (paged) {
-    if (rope) hipLaunchKernelGGL((prefill_lds2_kernel<G, true, true>), lgrid, lblock, 0, st, a);
-    else hipLaunchKernelGGL((prefill_lds2_kernel<G, false, true>), lgrid, lblock, 0, st, a);
-  } else {
-    if (rope) hipLaunchKernelGGL((prefill_lds2_kernel<G, true, false>), lgrid, lblock, 0, st, a);
-    else hipLaunchKernelGGL((prefill_lds2_kernel<G, false, false>), lgrid, lblock, 0, st, a);
-  }
-  return (int)hipGetLastError();
+  a.snake = cus > 0 && lgrid.x > (unsigned)cus && lgrid.x <= 2u * (unsigned)cus ? cus : 0;
+  return launch_stream<2>(a, rope, paged, lgrid, st);
 }
 
 static int fill_common(Args& a, const void* q, const void* k, const void* v, const void* cos,
