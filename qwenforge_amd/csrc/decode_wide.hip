@@ -20,8 +20,8 @@
 // Measured on MI355X (kernel trace, 896/4864 widths, 1024 tokens of context),
 // us at B=12 / 32, with the torch projections' kernels at B=12 beside them:
 // QKV + RoPE + append 5.1 / 6.4 (norm 3.6 + GEMM 7.3 + append 4.0), o_proj
-// 4.9 / 5.1 (7.3 + add 4.0), gate/up 7.2 / 12.0 (norm 3.6 + GEMM 10 + silu and
-// product 8), down 7.2 / 9.5 (13.4 + add 4.0), lm_head 46 / 52 (54 + argmax 49).
+// 4.7 / 4.8 (7.3 + add 4.0), gate/up 6.3 / 8.9 (norm 3.6 + GEMM 10 + silu and
+// product 8), down 6.9 / 8.1 (13.4 + add 4.0), lm_head 46 / 52 (54 + argmax 49).
 // The first four are bound by launch latency and the round trip of their
 // loads (1.6-17 MB of weights at 0.4-2.4 TB/s), the lm_head by HBM (5.9 TB/s).
 //
@@ -600,13 +600,24 @@ extern "C" int qf_wide_qkv(const void* x, int64_t x_sb, const void* norm_w, floa
   return (int)hipGetLastError();
 }
 
-// k blocks per wave: 8 in flight (plus their activation operands) before a
-// row block is split between workgroups.
-constexpr int kGemvBlk = 8;
+// k blocks per wave: up to 8 in one workgroup per row block; longer rows are
+// split between workgroups at 5 per wave, so that 56 row blocks x 8 splits
+// stream the 4864-wide down projection (MI355X, weights past the MALL, us at
+// B=12 / 32: 5 blocks, 8 splits 6.73 / 7.88; 8 blocks, 5 splits 7.06 / 9.26; 4
+// blocks, 10 splits 7.39 / 8.98; 13 blocks, 3 splits 7.24 / 8.94).
+constexpr int kGemvBlk = 8, kSplitBlk = 5;
 
 extern "C" int qf_wide_splits(int K) {
   if (K < 32 || K % 32) return QF_ERR_UNSUPPORTED;
-  return (K / 32 + kNW * kGemvBlk - 1) / (kNW * kGemvBlk);
+  const int nkb = K / 32, per = nkb <= kNW * kGemvBlk ? kGemvBlk : kSplitBlk;
+  return (nkb + kNW * per - 1) / (kNW * per);
+}
+
+template <int kBlk, bool kSplit>
+static void launch_gemv(const WideGemvArgs& a, hipStream_t st) {
+  const dim3 grid(a.N / 16, a.splits), block(kNT);
+  if (a.B <= 16) hipLaunchKernelGGL((wide_gemv_kernel<1, kBlk, kSplit>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((wide_gemv_kernel<2, kBlk, kSplit>), grid, block, 0, st, a);
 }
 
 extern "C" int qf_wide_gemv_residual(const void* inp, int64_t in_sb, const void* w, void* hidden,
@@ -625,14 +636,12 @@ extern "C" int qf_wide_gemv_residual(const void* inp, int64_t in_sb, const void*
   a.part = part; a.ticket = ticket;
   a.B = B; a.K = K; a.N = N; a.splits = splits;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid(N / 16, splits), block(kNT);
-  if (splits == 1) {
-    if (B <= 16) hipLaunchKernelGGL((wide_gemv_kernel<1, kGemvBlk, false>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((wide_gemv_kernel<2, kGemvBlk, false>), grid, block, 0, st, a);
-  } else {
-    if (B <= 16) hipLaunchKernelGGL((wide_gemv_kernel<1, kGemvBlk, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((wide_gemv_kernel<2, kGemvBlk, true>), grid, block, 0, st, a);
-  }
+  // A wave loads kBlk blocks whatever its share is, so o_proj's 28 take the
+  // 7-block form (3.82 us at B=12 against 4.05 with 8).
+  const int per = (K / 32 + kNW * splits - 1) / (kNW * splits);
+  if (splits > 1) launch_gemv<kSplitBlk, true>(a, st);
+  else if (per <= 7) launch_gemv<7, false>(a, st);
+  else launch_gemv<kGemvBlk, false>(a, st);
   return (int)hipGetLastError();
 }
 
@@ -650,7 +659,11 @@ extern "C" int qf_wide_gate_up(const void* x, int64_t x_sb, const void* norm_w, 
   a.h = static_cast<f16*>(h_out); a.h_sb = ho_sb;
   a.B = B; a.K = hidden; a.I = I;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  constexpr int kRB = 2;
+  // Three row blocks per workgroup: the 608 of Qwen2.5-0.5B then take 203
+  // workgroups, one round of the CUs, and the rows are staged a third as often
+  // (MI355X, weights past the MALL, us for 1 / 2 / 3 / 4 blocks: B=12 6.50 /
+  // 6.64 / 5.70 / 6.30, B=32 10.5 / 11.5 / 8.4 / 9.1).
+  constexpr int kRB = 3;
   const dim3 grid((I / 8 + kRB - 1) / kRB), block(kNT);
   QF_WIDE_DISPATCH(B, wide_gate_up_kernel, kRB)
   return (int)hipGetLastError();
