@@ -163,47 +163,6 @@ __device__ __forceinline__ void plain_finish(const f16x8 (&v)[XP], int C, int NB
 }
 
 // ---------------------------------------------------------------------------
-struct QkvArgs {
-  const f16* x;
-  int64_t x_sb;
-  const int64_t* token;
-  f16* hidden_out;
-  int64_t ho_sb;
-  const f16* norm_w;
-  float eps;
-  const f16* w;
-  const f16* bias;
-  const f16* cos;
-  const f16* sin;
-  int64_t cs_sb;
-  // Positions mode (cos == nullptr): row b's angle for frequency i is
-  // float(pos[b]) * inv_freq[i], and cos/sin are evaluated here in fp32 and
-  // rounded to fp16 -- bit-identical to the torch table (SE:910-915) that
-  // table mode reads.
-  const int64_t* pos;
-  const float* inv_freq;
-  f16* kc;
-  int64_t kc_sb, kc_sh, kc_sn;
-  f16* vc;
-  int64_t vc_sb, vc_sh, vc_sn;
-  const int64_t* write_index;
-  f16* q_out;
-  int64_t qo_sb, qo_sh;
-  int K, QH, KVH, cap, n_pairs;
-  // Paged caches: kc/vc are page pools (page strides kc_sb/vc_sb); row b
-  // appends at logical slot slots[b * slot_sb], in page
-  // table[b * t_sb + (slot >> log2p)].  cap = pages per row << log2p.
-  const int32_t* table;
-  int64_t t_sb;
-  int log2p, n_pages;
-  const int64_t* slots;
-  int64_t slot_sb;
-};
-static_assert(covers_lines(sizeof(QkvArgs), {offsetof(QkvArgs, x), offsetof(QkvArgs, bias),
-                                             offsetof(QkvArgs, write_index), offsetof(QkvArgs, K),
-                                             offsetof(QkvArgs, slots)}),
-              "touch_arg_lines fields cover every line");
-
 // One wave per (head, d) rotate-half pair: rows head*64 + d and head*64 + d + 32.
 template <int NB, bool kPaged, bool kPos>
 __global__ __launch_bounds__(kNT) void rms_qkv_rope_append_kernel(QkvArgs a) {
@@ -588,17 +547,6 @@ __global__ __launch_bounds__(kNT) void attn_merge_gemv_residual_kernel(MergeArgs
 }
 
 // ---------------------------------------------------------------------------
-struct GateUpArgs {
-  const f16* x;
-  int64_t x_sb;
-  const f16* norm_w;
-  float eps;
-  const f16* w;
-  f16* h;
-  int64_t h_sb;
-  int K, I;
-};
-
 // Each wave owns PW SwiGLU pairs (gate row j, up row I + j).
 template <int NB, int PW>
 __global__ __launch_bounds__(kNT) void rms_gate_up_swiglu_kernel(GateUpArgs a) {
@@ -694,7 +642,8 @@ __device__ __forceinline__ f32x4 tile_mfma(const f16x8 (&wa)[NBLK], const f16* x
 // matching up row (+ I) for i >= 2, so C registers t (gate) and t + 2 (up)
 // of lane l are one SwiGLU pair: lane l finishes outputs 8 rb + 2 (l >> 4)
 // + {0, 1} of batch row l & 15.  KS waves split a row block's k range and
-// add their partial tiles in LDS.
+// add their partial tiles in LDS.  One and two batch rows; from three the row-per-
+// wave staging of decode_wide.hip is the faster form.
 constexpr int kGuKS = 4;                             // k splits per row block
 constexpr int kGuBlk = kMaxNormK / 32 / kGuKS;       // k blocks per wave (max)
 
@@ -780,124 +729,6 @@ __global__ __launch_bounds__(kNT) void attn_merge_o_proj_mfma_kernel(MergeArgs a
 #pragma unroll
   for (int i = 0; i < 4; ++i) o[i] = (f16)((float)res[i] + (float)(f16)acc[i]);
   *reinterpret_cast<f16x4*>(hp) = o;
-}
-
-// QKV + bias + RoPE + KV append.  Packing QF_PACK_ROPE makes row block
-// rb = 4 head + c hold, in MFMA row r = 4g + i, row 64 head + d (i < 2) and
-// row 64 head + d + 32 (i >= 2) with d = 8c + 2g + (i & 1): lane l's C
-// registers t and t + 2 are the rotate-half pair of d = 8c + 2 (l >> 4) + t
-// for batch row l & 15, so bias, RoPE and the append run in the lane.
-constexpr int kQkvKS = 4;
-constexpr int kQkvBlk = kMaxNormK / 32 / kQkvKS;
-
-template <int NB, bool kPaged, bool kPos>
-__global__ __launch_bounds__(kNT) void rms_qkv_rope_append_mfma_kernel(QkvArgs a) {
-  __shared__ __attribute__((aligned(16))) f16 xs[NB * kMaxNormK];
-  __shared__ float red[kNW * NB];
-  __shared__ f32x4 part[kNW][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int K = touch_arg_lines(a.K, a.x, a.bias, a.write_index, a.slots), nkb = K / 32;
-  const int per = (nkb + kQkvKS - 1) / kQkvKS;
-  const int kp = w % kQkvKS;
-  const int nrb = (a.QH + 2 * a.KVH) * 4;
-  const int rb = min((int)blockIdx.x * (kNW / kQkvKS) + w / kQkvKS, nrb - 1);
-  const int kb0 = kp * per, n = min(per, nkb - kb0);
-  const f16* rows[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-    rows[b] = a.x + (a.token != nullptr ? a.token[b] : (int64_t)b) * a.x_sb;
-  RmsStage<NB> st;
-  rms_load<NB>(st, rows, K, a.norm_w);
-  // Epilogue operands, loaded now so their latency hides under the weights'.
-  const int col = lane & 15, q = lane >> 4;
-  const int be = min(col, NB - 1);
-  const int head = rb >> 2;
-  const int d0 = 8 * (rb & 3) + 2 * q;  // this lane's pair dims d0, d0 + 1 (and + 32)
-  const int64_t slot = kPaged ? a.slots[be * a.slot_sb] : a.write_index[0];
-  // Branch-free bias: without one, a weight element is read and dropped.
-  const bool has_bias = a.bias != nullptr;
-  const f16* bsrc = (has_bias ? a.bias : a.w) + 64 * head + d0;
-  float bias[2][2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const float lo = (float)bsrc[t], hi = (float)bsrc[t + 32];
-    bias[t][0] = has_bias ? lo : 0.f;
-    bias[t][1] = has_bias ? hi : 0.f;
-  }
-  float cs[2][4];  // per dim: cos_lo, sin_lo, cos_hi, sin_hi
-  float ang[2] = {0.f, 0.f};
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (kPos) {
-      ang[t] = (float)a.pos[be] * a.inv_freq[d0 + t];
-    } else {
-      const f16* cp = a.cos + be * a.cs_sb + d0 + t;
-      const f16* sp = a.sin + be * a.cs_sb + d0 + t;
-      cs[t][0] = (float)cp[0];
-      cs[t][1] = (float)sp[0];
-      cs[t][2] = (float)cp[32];
-      cs[t][3] = (float)sp[32];
-    }
-  }
-  f16x8 wa[kQkvBlk];
-#pragma unroll
-  for (int t = 0; t < kQkvBlk; ++t) wa[t] = tile_load(a.w, nkb, rb, min(kb0 + t, nkb - 1), lane);
-  // Destination slot offsets (kv head 0); the page lookup depends on the
-  // slot, so it is issued after the weights.
-  bool in_range = slot >= 0 && slot < a.cap;
-  int64_t kro, vro;
-  if (kPaged) {
-    const int64_t sl = in_range ? slot : 0;
-    const int page = a.table[be * a.t_sb + (sl >> a.log2p)];
-    in_range = in_range && page >= 0 && page < a.n_pages;
-    const int64_t prow = sl & ((1 << a.log2p) - 1);
-    kro = (int64_t)page * a.kc_sb + prow * a.kc_sn;
-    vro = (int64_t)page * a.vc_sb + prow * a.vc_sn;
-  } else {
-    kro = be * a.kc_sb + slot * a.kc_sn;
-    vro = be * a.vc_sb + slot * a.vc_sn;
-  }
-  if (kPos) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      cs[t][0] = cs[t][2] = (float)(f16)cosf(ang[t]);
-      cs[t][1] = cs[t][3] = (float)(f16)sinf(ang[t]);
-    }
-  }
-  f16* raw = (a.token != nullptr && blockIdx.x == 0) ? a.hidden_out : nullptr;
-  rms_finish<NB>(st, K, a.eps, xs, red, raw, a.ho_sb);
-  f32x4 acc = tile_mfma<NB, kQkvBlk>(wa, xs, K, kb0, n, lane);
-  if (kp != 0) part[w][lane] = acc;
-  __syncthreads();
-  if (kp != 0) return;
-#pragma unroll
-  for (int s = 1; s < kQkvKS; ++s) acc += part[w + s][lane];
-  const int rb_raw = (int)blockIdx.x * (kNW / kQkvKS) + w / kQkvKS;
-  if (col >= NB || rb_raw >= nrb) return;
-  const int b = col;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int d = d0 + t;
-    const float lo = (float)(f16)(acc[t] + bias[t][0]);
-    const float hi = (float)(f16)(acc[t + 2] + bias[t][1]);
-    if (head < a.QH + a.KVH) {
-      f16 olo, ohi;
-      rope1(lo, hi, cs[t][0], cs[t][1], cs[t][2], cs[t][3], olo, ohi);
-      if (head < a.QH) {
-        f16* qo = a.q_out + b * a.qo_sb + head * a.qo_sh;
-        qo[d] = olo;
-        qo[d + 32] = ohi;
-      } else if (in_range) {
-        f16* kd = a.kc + kro + (head - a.QH) * a.kc_sh;
-        kd[d] = olo;
-        kd[d + 32] = ohi;
-      }
-    } else if (in_range) {
-      f16* vd = a.vc + vro + (head - a.QH - a.KVH) * a.vc_sh;
-      vd[d] = (f16)lo;
-      vd[d + 32] = (f16)hi;
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1265,20 +1096,15 @@ extern "C" int qf_rms_qkv_rope_append(const void* x, int64_t x_sb, const int64_t
   a.vc = static_cast<f16*>(v_cache); a.vc_sb = vc_sb; a.vc_sh = vc_sh; a.vc_sn = vc_sn;
   a.write_index = write_index;
   a.q_out = static_cast<f16*>(q_out); a.qo_sb = qo_sb; a.qo_sh = qo_sh;
-  a.K = hidden; a.QH = QH; a.KVH = KVH; a.cap = cap;
+  a.K = hidden; a.QH = QH; a.KVH = KVH; a.cap = cap; a.B = B;
   a.n_pairs = (QH + 2 * KVH) * (kHeadDim / 2);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid((a.n_pairs + kNW - 1) / kNW), block(kNT);
   const size_t shm = 0;
   if (w_layout == QF_W_TILES) {
     if (hidden % 32) return QF_ERR_UNSUPPORTED;
-    const dim3 tgrid(((QH + 2 * KVH) * 4 + kNW / kQkvKS - 1) / (kNW / kQkvKS));
-    const dim3& grid = tgrid;
-    if (rope_mode == 1) {
-      QF_DISPATCH_B(B, rms_qkv_rope_append_mfma_kernel, false, true)
-    } else {
-      QF_DISPATCH_B(B, rms_qkv_rope_append_mfma_kernel, false, false)
-    }
+    a.slots = write_index;
+    launch_qkv_tiles(a, false, rope_mode == 1, st);
   } else if (rope_mode == 1) {
     QF_DISPATCH_B(B, rms_qkv_rope_append_kernel, false, true)
   } else {
@@ -1325,6 +1151,7 @@ extern "C" int qf_rms_qkv_rope_append_paged(const void* x, int64_t x_sb, const i
   a.write_index = nullptr;
   a.q_out = static_cast<f16*>(q_out); a.qo_sb = qo_sb; a.qo_sh = qo_sh;
   a.K = hidden; a.QH = QH; a.KVH = KVH; a.cap = pages_per_row * page_size;
+  a.B = B;
   a.n_pairs = (QH + 2 * KVH) * (kHeadDim / 2);
   a.table = block_table; a.t_sb = bt_sb; a.log2p = l2; a.n_pages = n_pages;
   a.slots = slots; a.slot_sb = slot_sb;
@@ -1333,13 +1160,7 @@ extern "C" int qf_rms_qkv_rope_append_paged(const void* x, int64_t x_sb, const i
   const size_t shm = 0;
   if (w_layout == QF_W_TILES) {
     if (hidden % 32) return QF_ERR_UNSUPPORTED;
-    const dim3 tgrid(((QH + 2 * KVH) * 4 + kNW / kQkvKS - 1) / (kNW / kQkvKS));
-    const dim3& grid = tgrid;
-    if (rope_mode == 1) {
-      QF_DISPATCH_B(B, rms_qkv_rope_append_mfma_kernel, true, true)
-    } else {
-      QF_DISPATCH_B(B, rms_qkv_rope_append_mfma_kernel, true, false)
-    }
+    launch_qkv_tiles(a, true, rope_mode == 1, st);
   } else if (rope_mode == 1) {
     QF_DISPATCH_B(B, rms_qkv_rope_append_kernel, true, true)
   } else {
@@ -1430,7 +1251,7 @@ extern "C" int qf_rms_gate_up_swiglu(const void* x, int64_t x_sb, const void* no
   a.norm_w = static_cast<const f16*>(norm_w); a.eps = eps;
   a.w = static_cast<const f16*>(w_gate_up);
   a.h = static_cast<f16*>(h_out); a.h_sb = ho_sb;
-  a.K = hidden; a.I = I;
+  a.K = hidden; a.I = I; a.B = B;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 block(kNT);
   const size_t shm = 0;
@@ -1438,7 +1259,9 @@ extern "C" int qf_rms_gate_up_swiglu(const void* x, int64_t x_sb, const void* no
     // 8 SwiGLU pairs per row block, kNW / kGuKS row blocks per workgroup.
     if (hidden % 32 || I % 8) return QF_ERR_UNSUPPORTED;
     const dim3 grid((I / 8 + kNW / kGuKS - 1) / (kNW / kGuKS));
-    QF_DISPATCH_B(B, rms_gate_up_swiglu_mfma_kernel)
+    if (B == 1) hipLaunchKernelGGL(rms_gate_up_swiglu_mfma_kernel<1>, grid, block, shm, st, a);
+    else if (B == 2) hipLaunchKernelGGL(rms_gate_up_swiglu_mfma_kernel<2>, grid, block, shm, st, a);
+    else launch_gate_up_tiles(a, st);
   } else {
     constexpr int PW = 2;
     const dim3 grid((I + kNW * PW - 1) / (kNW * PW));

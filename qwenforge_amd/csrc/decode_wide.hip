@@ -1,4 +1,5 @@
-// Decode-step projections for 5..32 batch rows (gfx950 / MI355X).
+// Decode-step projections on packed weight tiles for up to 32 batch rows
+// (gfx950 / MI355X): QKV from one row on, gate/up from three, the others from five.
 //
 // Below 16 rows an MFMA column is still mostly idle work, so the cost of a
 // projection stays streaming its weight once, as at 1..4 rows
@@ -40,7 +41,8 @@ constexpr int kNormBlk = kMaxNormK / 32 / kNW;  // k blocks per wave of a normal
 constexpr int col_blocks(int rows_per_wave) { return rows_per_wave > 4 ? 2 : 1; }
 
 // RMSNorm staging, fp32 math and one rounding: wave w owns rows w, w + 4, ...
-// Rows past B re-read row B - 1 (their columns are never stored).  Split so
+// Rows past B re-read row B - 1 (their columns are never stored); `token`
+// gathers the rows of an embedding table.  Split so
 // that the caller's weight loads go out in between.
 template <int kRows>
 struct WideStage {
@@ -50,13 +52,14 @@ struct WideStage {
 
 template <int kRows>
 __device__ __forceinline__ void wide_load(WideStage<kRows>& st, const f16* __restrict__ x,
-                                          int64_t x_sb, int B, int C,
-                                          const f16* __restrict__ nw) {
+                                          int64_t x_sb, int B, int C, const f16* __restrict__ nw,
+                                          const int64_t* token = nullptr) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int c0 = min(lane, C - 1), c1 = min(lane + 64, C - 1);
 #pragma unroll
   for (int i = 0; i < kRows; ++i) {
-    const f16* row = x + (int64_t)min(w + kNW * i, B - 1) * x_sb;
+    const int r = min(w + kNW * i, B - 1);
+    const f16* row = x + (token != nullptr ? token[r] : (int64_t)r) * x_sb;
     st.x[i][0] = load16(row + 8 * c0);
     st.x[i][1] = load16(row + 8 * c1);
   }
@@ -115,46 +118,20 @@ __device__ __forceinline__ void wide_mfma(const f16x8 (&wa)[kBlk], const f16* xs
 }
 
 // ---------------------------------------------------------------------------
-struct WideQkvArgs {
-  const f16* x;
-  int64_t x_sb;
-  const f16* norm_w;
-  float eps;
-  const f16* w;
-  const f16* bias;
-  const int64_t* pos;
-  const float* inv_freq;
-  f16* kc;
-  int64_t kc_sb, kc_sh, kc_sn;
-  f16* vc;
-  int64_t vc_sb, vc_sh, vc_sn;
-  const int64_t* slots;
-  int64_t slot_sb;
-  f16* q_out;
-  int64_t qo_sb, qo_sh;
-  int B, K, QH, KVH, cap;
-  const int32_t* table;
-  int64_t t_sb;
-  int log2p, n_pages;
-};
-static_assert(covers_lines(sizeof(WideQkvArgs),
-                           {offsetof(WideQkvArgs, x), offsetof(WideQkvArgs, kc),
-                            offsetof(WideQkvArgs, K), offsetof(WideQkvArgs, table)}),
-              "touch_arg_lines fields cover every line");
-
 // One 16-row block (QF_PACK_ROPE: rotate-half pairs in C registers t and
 // t + 2 of a lane) per workgroup; wave c < NC finishes column block c.
-template <int kRows, bool kPaged>
-__global__ __launch_bounds__(kNT) void wide_qkv_kernel(WideQkvArgs a) {
+template <int kRows, bool kPaged, bool kPos>
+__global__ __launch_bounds__(kNT) void wide_qkv_kernel(QkvArgs a) {
   constexpr int NC = col_blocks(kRows);
   __shared__ __attribute__((aligned(16))) f16 xs[kNW * kRows * (kMaxNormK + kPad)];
   __shared__ f32x4 part[kNW][NC][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int K = touch_arg_lines(a.K, a.x, a.kc, a.table), nkb = K / 32;
+  const int K = touch_arg_lines(a.K, a.x, a.bias, a.write_index, a.slots), nkb = K / 32;
   const int per = (nkb + kNW - 1) / kNW, kb0 = w * per, n = min(per, nkb - kb0);
   const int rb = blockIdx.x;
   WideStage<kRows> st;
-  wide_load<kRows>(st, a.x, a.x_sb, a.B, K / 8, a.norm_w);
+  // Gathered rows: the 1..4-row entry points only.
+  wide_load<kRows>(st, a.x, a.x_sb, a.B, K / 8, a.norm_w, kRows == 1 ? a.token : nullptr);
   // Epilogue operands of this wave's column block, loaded ahead of the weights.
   const int q = lane >> 4, col = 16 * min(w, NC - 1) + (lane & 15), be = min(col, a.B - 1);
   const int head = rb >> 2, d0 = 8 * (rb & 3) + 2 * q;
@@ -162,12 +139,22 @@ __global__ __launch_bounds__(kNT) void wide_qkv_kernel(WideQkvArgs a) {
   const bool has_bias = a.bias != nullptr;
   const f16* bsrc = (has_bias ? a.bias : a.w) + 64 * head + d0;
   float bias[2][2], ang[2];
+  float cs[2][4];  // per dim: cos_lo, sin_lo, cos_hi, sin_hi
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const float lo = (float)bsrc[t], hi = (float)bsrc[t + 32];
     bias[t][0] = has_bias ? lo : 0.f;
     bias[t][1] = has_bias ? hi : 0.f;
-    ang[t] = (float)a.pos[be] * a.inv_freq[d0 + t];
+    if (kPos) {
+      ang[t] = (float)a.pos[be] * a.inv_freq[d0 + t];
+    } else {
+      const f16* cp = a.cos + be * a.cs_sb + d0 + t;
+      const f16* sp = a.sin + be * a.cs_sb + d0 + t;
+      cs[t][0] = (float)cp[0];
+      cs[t][1] = (float)sp[0];
+      cs[t][2] = (float)cp[32];
+      cs[t][3] = (float)sp[32];
+    }
   }
   f16x8 wa[kNormBlk];
 #pragma unroll
@@ -185,11 +172,21 @@ __global__ __launch_bounds__(kNT) void wide_qkv_kernel(WideQkvArgs a) {
     kro = be * a.kc_sb + slot * a.kc_sn;
     vro = be * a.vc_sb + slot * a.vc_sn;
   }
-  float cs[2], sn[2];
+  if (kPos) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    cs[t] = (float)(f16)cosf(ang[t]);
-    sn[t] = (float)(f16)sinf(ang[t]);
+    for (int t = 0; t < 2; ++t) {
+      cs[t][0] = cs[t][2] = (float)(f16)cosf(ang[t]);
+      cs[t][1] = cs[t][3] = (float)(f16)sinf(ang[t]);
+    }
+  }
+  if (kRows == 1 && a.token != nullptr && a.hidden_out != nullptr && blockIdx.x == 0) {
+    // The gathered embedding rows, as the residual stream.
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (w + kNW * i < a.B && lane + 64 * h < K / 8)
+          store16(a.hidden_out + (w + kNW * i) * a.ho_sb + 8 * (lane + 64 * h), st.x[i][h]);
   }
   wide_finish<kRows>(st, K, a.eps, xs);
   f32x4 acc[NC];
@@ -208,7 +205,7 @@ __global__ __launch_bounds__(kNT) void wide_qkv_kernel(WideQkvArgs a) {
     const float hi = (float)(f16)(sum[t + 2] + bias[t][1]);
     if (head < a.QH + a.KVH) {
       f16 olo, ohi;
-      rope1(lo, hi, cs[t], sn[t], cs[t], sn[t], olo, ohi);
+      rope1(lo, hi, cs[t][0], cs[t][1], cs[t][2], cs[t][3], olo, ohi);
       if (head < a.QH) {
         f16* qo = a.q_out + col * a.qo_sb + head * a.qo_sh;
         qo[d] = olo;
@@ -333,21 +330,10 @@ __global__ __launch_bounds__(kNT) void wide_gemv_kernel(WideGemvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-struct WideGateUpArgs {
-  const f16* x;
-  int64_t x_sb;
-  const f16* norm_w;
-  float eps;
-  const f16* w;
-  f16* h;
-  int64_t h_sb;
-  int B, K, I;
-};
-
 // Gate/up + SwiGLU (QF_PACK_SWIGLU: gate and up of a pair in C registers t
 // and t + 2 of a lane), kRB row blocks per workgroup.
 template <int kRows, int kRB>
-__global__ __launch_bounds__(kNT) void wide_gate_up_kernel(WideGateUpArgs a) {
+__global__ __launch_bounds__(kNT) void wide_gate_up_kernel(GateUpArgs a) {
   constexpr int NC = col_blocks(kRows);
   __shared__ __attribute__((aligned(16))) f16 xs[kNW * kRows * (kMaxNormK + kPad)];
   __shared__ f32x4 part[kNW][kRB * NC][64];
@@ -562,6 +548,38 @@ static bool wide_rows(int B) { return B >= 5 && B <= QF_WIDE_MAX_B; }
     default: hipLaunchKernelGGL((KERNEL<8, ##__VA_ARGS__>), grid, block, 0, st, a); break;       \
   }
 
+// One row per wave up to 4 rows.  Measured on MI355X (weights past the MALL):
+// at B=4 3.47 us against 4.04 for the 1..4-row form this replaced, whose
+// workgroup reduced every row together and read its operands with LDS bank
+// conflicts; B=2 3.48.
+void qf::step::launch_qkv_tiles(const QkvArgs& a, bool paged, bool positions, hipStream_t st) {
+  const dim3 grid((a.QH + 2 * a.KVH) * 4), block(kNT);
+  if (a.B > 4) {  // positions only: the 5..32-row entry point takes no tables
+    if (paged) { QF_WIDE_DISPATCH(a.B, wide_qkv_kernel, true, true) }
+    else { QF_WIDE_DISPATCH(a.B, wide_qkv_kernel, false, true) }
+  } else if (positions) {
+    if (paged) hipLaunchKernelGGL((wide_qkv_kernel<1, true, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((wide_qkv_kernel<1, false, true>), grid, block, 0, st, a);
+  } else {
+    if (paged) hipLaunchKernelGGL((wide_qkv_kernel<1, true, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((wide_qkv_kernel<1, false, false>), grid, block, 0, st, a);
+  }
+}
+
+// From 3 rows (below, re-reading the last row in the spare ones costs more than
+// it saves: B=2 5.75 us against 5.46 for rms_gate_up_swiglu_mfma_kernel).
+// Three row blocks per workgroup: the 608 of Qwen2.5-0.5B then take 203
+// workgroups, one round of the CUs, and the rows are staged a third as often
+// (MI355X, weights past the MALL, us for 1 / 2 / 3 / 4 blocks: B=12 6.50 /
+// 6.64 / 5.70 / 6.30, B=32 10.5 / 11.5 / 8.4 / 9.1).  Up to 8 rows the two-row
+// instance: at B=4 5.53 against 6.28 with one row per wave, and 6.03 for
+// rms_gate_up_swiglu_mfma_kernel (B=3 5.54 against 5.78).
+void qf::step::launch_gate_up_tiles(const GateUpArgs& a, hipStream_t st) {
+  constexpr int kRB = 3;
+  const dim3 grid((a.I / 8 + kRB - 1) / kRB), block(kNT);
+  QF_WIDE_DISPATCH(a.B < 5 ? 5 : a.B, wide_gate_up_kernel, kRB)
+}
+
 extern "C" int qf_wide_qkv(const void* x, int64_t x_sb, const void* norm_w, float eps,
                            const void* w_qkv, const void* bias, const int64_t* pos,
                            const float* inv_freq, void* k_cache, int64_t kc_sb, int64_t kc_sh,
@@ -576,7 +594,7 @@ extern "C" int qf_wide_qkv(const void* x, int64_t x_sb, const void* norm_w, floa
     return QF_ERR_INVALID_ARG;
   if (QH < 1 || KVH < 1 || cap < 1) return QF_ERR_INVALID_ARG;
   if (!al16(x) || !al16(norm_w) || !al16(w_qkv) || (x_sb & 7)) return QF_ERR_INVALID_ARG;
-  WideQkvArgs a;
+  QkvArgs a = {};
   a.x = static_cast<const f16*>(x); a.x_sb = x_sb;
   a.norm_w = static_cast<const f16*>(norm_w); a.eps = eps;
   a.w = static_cast<const f16*>(w_qkv); a.bias = static_cast<const f16*>(bias);
@@ -586,17 +604,13 @@ extern "C" int qf_wide_qkv(const void* x, int64_t x_sb, const void* norm_w, floa
   a.slots = slots; a.slot_sb = slot_sb;
   a.q_out = static_cast<f16*>(q_out); a.qo_sb = qo_sb; a.qo_sh = qo_sh;
   a.B = B; a.K = hidden; a.QH = QH; a.KVH = KVH; a.cap = cap;
-  a.table = block_table; a.t_sb = bt_sb; a.log2p = 0; a.n_pages = n_pages;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid((QH + 2 * KVH) * 4), block(kNT);
+  a.table = block_table; a.t_sb = bt_sb; a.n_pages = n_pages;
   if (block_table != nullptr) {
     a.log2p = page_log2(page_size, pages_per_row, n_pages);
     if (a.log2p < 0) return QF_ERR_UNSUPPORTED;
     if (bt_sb < pages_per_row || cap != pages_per_row * page_size) return QF_ERR_INVALID_ARG;
-    QF_WIDE_DISPATCH(B, wide_qkv_kernel, true)
-  } else {
-    QF_WIDE_DISPATCH(B, wide_qkv_kernel, false)
   }
+  launch_qkv_tiles(a, block_table != nullptr, true, static_cast<hipStream_t>(stream));
   return (int)hipGetLastError();
 }
 
@@ -652,20 +666,13 @@ extern "C" int qf_wide_gate_up(const void* x, int64_t x_sb, const void* norm_w, 
     return QF_ERR_UNSUPPORTED;
   if (!x || !norm_w || !w_gate_up || !h_out) return QF_ERR_INVALID_ARG;
   if (!al16(x) || !al16(norm_w) || !al16(w_gate_up) || (x_sb & 7)) return QF_ERR_INVALID_ARG;
-  WideGateUpArgs a;
+  GateUpArgs a;
   a.x = static_cast<const f16*>(x); a.x_sb = x_sb;
   a.norm_w = static_cast<const f16*>(norm_w); a.eps = eps;
   a.w = static_cast<const f16*>(w_gate_up);
   a.h = static_cast<f16*>(h_out); a.h_sb = ho_sb;
   a.B = B; a.K = hidden; a.I = I;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  // Three row blocks per workgroup: the 608 of Qwen2.5-0.5B then take 203
-  // workgroups, one round of the CUs, and the rows are staged a third as often
-  // (MI355X, weights past the MALL, us for 1 / 2 / 3 / 4 blocks: B=12 6.50 /
-  // 6.64 / 5.70 / 6.30, B=32 10.5 / 11.5 / 8.4 / 9.1).
-  constexpr int kRB = 3;
-  const dim3 grid((I / 8 + kRB - 1) / kRB), block(kNT);
-  QF_WIDE_DISPATCH(B, wide_gate_up_kernel, kRB)
+  launch_gate_up_tiles(a, static_cast<hipStream_t>(stream));
   return (int)hipGetLastError();
 }
 

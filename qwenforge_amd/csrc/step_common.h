@@ -68,5 +68,64 @@ __device__ __forceinline__ uint64_t argmax_key(f16 v, int index) {
   return ((uint64_t)ord << 32) | (uint64_t)(0xFFFFFFFFu - (unsigned)index);
 }
 
+// Arguments of the QKV kernels (row-major and tiles).
+struct QkvArgs {
+  const f16* x;
+  int64_t x_sb;
+  const int64_t* token;
+  f16* hidden_out;
+  int64_t ho_sb;
+  const f16* norm_w;
+  float eps;
+  const f16* w;
+  const f16* bias;
+  const f16* cos;
+  const f16* sin;
+  int64_t cs_sb;
+  // Positions mode (cos == nullptr): row b's angle for frequency i is
+  // float(pos[b]) * inv_freq[i], and cos/sin are evaluated here in fp32 and
+  // rounded to fp16 -- bit-identical to the torch table (SE:910-915) that
+  // table mode reads.
+  const int64_t* pos;
+  const float* inv_freq;
+  f16* kc;
+  int64_t kc_sb, kc_sh, kc_sn;
+  f16* vc;
+  int64_t vc_sb, vc_sh, vc_sn;
+  const int64_t* write_index;
+  f16* q_out;
+  int64_t qo_sb, qo_sh;
+  int K, QH, KVH, cap, n_pairs, B;
+  // Paged caches: kc/vc are page pools (page strides kc_sb/vc_sb); row b
+  // appends at logical slot slots[b * slot_sb], in page
+  // table[b * t_sb + (slot >> log2p)].  cap = pages per row << log2p.
+  const int32_t* table;
+  int64_t t_sb;
+  int log2p, n_pages;
+  const int64_t* slots;  // the tile kernels' dense form too: write_index, stride 0
+  int64_t slot_sb;
+};
+static_assert(covers_lines(sizeof(QkvArgs), {offsetof(QkvArgs, x), offsetof(QkvArgs, bias),
+                                             offsetof(QkvArgs, write_index), offsetof(QkvArgs, K),
+                                             offsetof(QkvArgs, slots)}),
+              "touch_arg_lines fields cover every line");
+
+// Arguments of the gate/up kernels.
+struct GateUpArgs {
+  const f16* x;
+  int64_t x_sb;
+  const f16* norm_w;
+  float eps;
+  const f16* w;
+  f16* h;
+  int64_t h_sb;
+  int K, I, B;
+};
+
+// The matrix-core forms of decode_wide.hip (QKV 1..32 rows, gate/up 3..32);
+// a.B holds the rows.
+void launch_qkv_tiles(const QkvArgs& a, bool paged, bool positions, hipStream_t st);
+void launch_gate_up_tiles(const GateUpArgs& a, hipStream_t st);
+
 }  // namespace step
 }  // namespace qf
