@@ -85,13 +85,18 @@ int qf_abi_version(void);
  *          With splits = 1 one workgroup per (b, kv head) covers every slot,
  *          merges its waves in LDS and writes `out` itself: acc, m, l and the
  *          ticket are not read or written.
+ *          With a ticket, kv_last per row, no bias, splits <= 8 and
+ *          cap >= 192 * splits the B * splits workgroups of a kv head are
+ *          shared out by the rows' lengths instead (up to 16 splits for a
+ *          long row), so a row's rounding then depends on the other rows'
+ *          bounds too; the partials of one kv head lie together.
  *   ticket NULL: the merge runs as a second kernel (reference two-launch
  *          shape).  Non-NULL: int32[B*KVH], one counter per (b, kv head),
  *          zero-filled once by the caller; the merge runs inside the same
  *          launch: every workgroup of a (b, h) stores its partial, waits for
  *          the stores to complete and increments the counter, and the
- *          workgroup that completes the count (splits increments) merges all
- *          `splits` partials, writes the output and re-arms the counter to 0,
+ *          workgroup that completes the count (one increment a split) merges all
+ *          partials of the row, writes the output and re-arms the counter to 0,
  *          so the same ticket serves every later call.  Calls that share a
  *          ticket or the partials must not overlap in time.
  *   out    (B, KVH, G, D) fp16, strides o_sb, o_sh, o_sg.

@@ -50,7 +50,9 @@ constexpr int kVtStride = 36;   // LDS row stride (halves) of a transposed V til
 constexpr int kMaxG = 16;
 
 // kPartialCap: kPartial over the capacity split (split_range<true>).
-enum Mode { kDirect = 0, kPartial = 1, kFused = 2, kPartialCap = 3 };
+// kFusedRows: kFused with the workgroups shared out by the rows' lengths
+// (row_share).
+enum Mode { kDirect = 0, kPartial = 1, kFused = 2, kPartialCap = 3, kFusedRows = 4 };
 
 // Merge mode of a call with `splits` partials; `ticket`: the caller passed
 // merge counters (single launch).
@@ -106,17 +108,68 @@ __device__ __forceinline__ void st_wt(float* p, float v) {
 // SE:851), so the ranges need no device load; kv_last then only masks (see
 // the kernel).  A compile-time choice: with a run-time one the ranges would
 // still wait for the load through a select.
-template <bool kCap>
-__device__ __forceinline__ void split_range(const DecodeArgs& a, int b, int s, int& lo, int& hi) {
-  int span = a.cap;
-  if (!kCap && a.kv_last != nullptr) {
-    const int64_t last = a.kv_last[(int64_t)b * a.kv_last_sb];
-    span = (int)(last + 1 < 0 ? 0 : (last + 1 > a.cap ? a.cap : last + 1));
-  }
-  int split_len = (span + a.splits - 1) / a.splits;
+__device__ __forceinline__ int valid_slots(const DecodeArgs& a, int64_t last) {
+  return (int)(last + 1 < 0 ? 0 : (last + 1 > a.cap ? a.cap : last + 1));
+}
+
+__device__ __forceinline__ void cut_range(int span, int splits, int s, int& lo, int& hi) {
+  int split_len = (span + splits - 1) / splits;
   split_len = (split_len + kTile - 1) / kTile * kTile;
   lo = s * split_len;
   hi = lo + split_len < span ? lo + split_len : span;
+}
+
+template <bool kCap>
+__device__ __forceinline__ void split_range(const DecodeArgs& a, int b, int s, int& lo, int& hi) {
+  int span = a.cap;
+  if (!kCap && a.kv_last != nullptr) span = valid_slots(a, a.kv_last[(int64_t)b * a.kv_last_sb]);
+  cut_range(span, a.splits, s, lo, hi);
+}
+
+// Inclusive sum over lanes 0 .. lane (DPP, no LDS).
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_add_int(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xF, false);
+}
+__device__ __forceinline__ int lane_scan(int v) {
+  v = dpp_add_int<0x111, 0xF>(v);  // row_shr:1
+  v = dpp_add_int<0x112, 0xF>(v);  // row_shr:2
+  v = dpp_add_int<0x114, 0xF>(v);  // row_shr:4
+  v = dpp_add_int<0x118, 0xF>(v);  // row_shr:8: sums within 16 lanes
+  v = dpp_add_int<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
+  return dpp_add_int<0x143, 0xC>(v);  // row_bcast:31 into rows 2, 3
+}
+
+// kFusedRows: the W = S * B workgroups of a kv head are shared out by length
+// instead of S to every row, so a long row among short ones gets more splits
+// and its waves the same number of tiles as everybody's.  Row r gets n_r = 1 +
+// floor(tiles_r (W - B) / tiles), at most kMaxRowSplits (one batch of the
+// merge; 32 measured 9.8 us against 8.9 on 9 paged rows of 100-4000 slots): sum
+// n_r <= W, and rows of equal length get S each.  Workgroup u of
+// the kv head takes split u - sum of the earlier rows' n; its partial lies in
+// slot u of the kv head's W (the scratch's B * S, in another order).  Lane r
+// < B <= 64 works out row r.  Returns false for a spare workgroup.
+constexpr int kMaxRowSplits = 16;
+struct RowShare {
+  int b, s, splits, span, base;
+};
+__device__ __forceinline__ bool row_share(const DecodeArgs& a, int u, RowShare& r) {
+  const int lane = threadIdx.x & 63;
+  const int64_t last = a.kv_last[(int64_t)min(lane, a.B - 1) * a.kv_last_sb];
+  const int span = lane < a.B ? valid_slots(a, last) : 0;
+  const unsigned tiles = (unsigned)(span + kTile - 1) / kTile;
+  const unsigned total = (unsigned)__builtin_amdgcn_readlane(lane_scan((int)tiles), 63);
+  // The host checks that the product fits 32 bits.
+  const unsigned more = tiles * (unsigned)(a.splits * a.B - a.B) / (total > 0u ? total : 1u);
+  const int n = lane < a.B ? min(1 + (int)more, kMaxRowSplits) : 0;
+  const int end = lane_scan(n);
+  const int row = __builtin_popcountll(__ballot(lane < a.B && end - n <= u)) - 1;
+  r.b = row;
+  r.splits = __builtin_amdgcn_readlane(n, row);
+  r.base = __builtin_amdgcn_readlane(end, row) - r.splits;
+  r.span = __builtin_amdgcn_readlane(span, row);
+  r.s = u - r.base;
+  return r.s < r.splits;
 }
 
 // (M, L, A) <- log-sum-exp merge of two partial states (m in natural-log
@@ -158,7 +211,8 @@ __device__ __forceinline__ void lse_merge_lanes(float& M, float& L, f32x4& A) {
   A = a0;
 }
 
-// Folds partials of query q of (b, h) = bh into the running state (M, L, A)
+// Folds the S partials of query q of one (b, h), the first in scratch slot
+// pbase, into the running state (M, L, A)
 // of dims 4*d4 .. +3, d4 = lane % 16.  The wave's four 16-lane rows hold the
 // consecutive subs sub0 + lane / 16 out of nsub; sub folds partials
 // j = sub + nsub * u, batch after batch of kB (j < S).  In a batch the wave
@@ -176,13 +230,12 @@ __device__ __forceinline__ void lse_merge_lanes(float& M, float& L, f32x4& A) {
 // kCoherent: sc1 loads, for partials that other workgroups of the same
 // launch stored with sc1 stores.
 template <int kB, bool kCoherent>
-__device__ __forceinline__ void fold_wave(const DecodeArgs& a, int bh, int q, int lane, int sub0,
-                                          int nsub, float& M, float& L, f32x4& A) {
+__device__ __forceinline__ void fold_wave(const DecodeArgs& a, int64_t pbase, int S, int q, int lane,
+                                          int sub0, int nsub, float& M, float& L, f32x4& A) {
   static_assert(4 * kB <= 64, "a batch's (m, l) must fit one load per lane");
-  const int G = a.G, S = a.splits;
+  const int G = a.G;
   const int s4 = lane >> 4, d4 = lane & 15, sub = sub0 + s4;
   constexpr int aux = kCoherent ? kSc1 : 0;
-  const int64_t pbase = (int64_t)bh * S;
   const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(a.acc + pbase * G * kD, (int64_t)S * G * kD * 4);
   const __amdgpu_buffer_rsrc_t rm = buffer_rsrc(a.m + pbase * G, (int64_t)S * G * 4);
   const __amdgpu_buffer_rsrc_t rl = buffer_rsrc(a.l + pbase * G, (int64_t)S * G * 4);
@@ -310,12 +363,20 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
   __shared__ float sm_ml[2][NW][kMaxG];
   __shared__ int sh_last;
 
-  const int s = blockIdx.x;
-  const int bh = blockIdx.y;
+  int s = blockIdx.x;
+  int bh = blockIdx.y;
   // The fields the first loads depend on (q, the kv_last bound, K/V and the
   // bias rows), one from each further line (acc, log2p).
   const int KVH = touch_arg_lines(a.KVH, a.q, a.v, a.bias, a.kv_last, a.kv_last_sb, a.acc, a.log2p);
-  const int b = bh / KVH, h = bh % KVH;
+  int b = bh / KVH;
+  const int h = bh % KVH;
+  RowShare share = {0, 0, 0, 0, 0};
+  if constexpr (kMode == kFusedRows) {
+    if (!row_share(a, b * a.splits + s, share)) return;
+    b = share.b;
+    s = share.s;
+    bh = b * KVH + h;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: tile math stays scalar
@@ -342,7 +403,8 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
 
   constexpr bool kCap = kMode == kPartialCap;
   int lo, hi;
-  split_range<kCap>(a, b, s, lo, hi);
+  if constexpr (kMode == kFusedRows) cut_range(share.span, share.splits, s, lo, hi);
+  else split_range<kCap>(a, b, s, lo, hi);
   // kCap: kv_last only masks.  It is read with a vector load (a VGPR
   // address), issued with the q loads ahead of the first tile's, and first
   // used in the first tile's compute: the wait for it is then an in-order
@@ -544,8 +606,11 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
   for (int t = 0; t < 4; ++t) sm_o(w)[t * 64 + lane] = o[t];
   __syncthreads();
 
-  const int S = a.splits, G = a.G;
-  const int64_t part = (int64_t)bh * S + s;
+  constexpr bool kRows = kMode == kFusedRows;
+  const int S = kRows ? share.splits : a.splits, G = a.G;
+  const int64_t pbase =
+      kRows ? (int64_t)h * a.splits * a.B + share.base : (int64_t)bh * a.splits;
+  const int64_t part = pbase + s;
   if (w < 4) {
     float mw[NW], wt[NW];
     float M = kNegInf;
@@ -593,7 +658,7 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
     }
   }
 
-  if (kMode == kFused) {
+  if (kMode == kFused || kRows) {
     // Publication.  The partial stores above are write-through (sc1) stores,
     // i.e. relaxed agent-scope atomic stores.  Each wave waits until its own
     // have been acknowledged (vmcnt counts stores on gfx9); after the barrier
@@ -615,8 +680,8 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
     for (int q = w; q < G; q += NW) {
       float Mq = kNegInf, Lq = 0.f;
       f32x4 Aq = {0.f, 0.f, 0.f, 0.f};
-      if (S <= 16) fold_wave<4, true>(a, bh, q, lane, 0, 4, Mq, Lq, Aq);
-      else fold_wave<8, true>(a, bh, q, lane, 0, 4, Mq, Lq, Aq);
+      if (S <= 16) fold_wave<4, true>(a, pbase, S, q, lane, 0, 4, Mq, Lq, Aq);
+      else fold_wave<8, true>(a, pbase, S, q, lane, 0, 4, Mq, Lq, Aq);
       lse_merge_lanes<false>(Mq, Lq, Aq);
       lse_merge_lanes<true>(Mq, Lq, Aq);
       if (lane < 16) store_out(a, bh, q, lane, Lq, Aq);
@@ -639,7 +704,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a) {
   const int d4 = lane & 15;
   float M = kNegInf, L = 0.f;
   f32x4 A = {0.f, 0.f, 0.f, 0.f};
-  fold_wave<8, false>(a, bh, q, lane, 4 * w, 16, M, L, A);
+  fold_wave<8, false>(a, (int64_t)bh * a.splits, a.splits, q, lane, 4 * w, 16, M, L, A);
   lse_merge_lanes<false>(M, L, A);
   lse_merge_lanes<true>(M, L, A);
   if (w > 0 && lane < 16) {
@@ -676,6 +741,9 @@ static void launch_split(const DecodeArgs& a, int mode, dim3 grid, hipStream_t s
   } else if (mode == kPartialCap) {
     if constexpr (!kPaged)
       hipLaunchKernelGGL((decode_split_kernel<NW, kBias, kPartialCap, false>), grid, block, 0, st, a);
+  } else if (mode == kFusedRows) {
+    if constexpr (kBias == kNoBias && NW <= 8)
+      hipLaunchKernelGGL((decode_split_kernel<NW, kBias, kFusedRows, kPaged>), grid, block, 0, st, a);
   } else if constexpr (kBias == kBiasVec && !kPaged) {
     launch_fused_vec(a, NW, grid, st);
   } else {
@@ -785,10 +853,26 @@ static int make_args(DecodeArgs& a, const void* q, int64_t q_sb, int64_t q_sh, i
 }
 
 
+// Whether a single-launch merge shares its workgroups out by the rows' lengths:
+// rows with bounds of their own (and no bias, which may mask anything), at most
+// eight splits a row and at least six tiles of capacity for each.  Measured on
+// MI355X, us per call, even / shared: paged 16 rows of 201-6007 slots 12.45 /
+// 10.42, 24 of 50-2800 10.59 / 9.50, 32 of 50-2000 10.52 / 9.24, equal rows
+// 13.84 / 13.94 (16 of 6000) and 11.46 / 11.31 (32 of 2000).  Outside the rule
+// working the shares out costs more than it saves: 9 rows of 100-4000 (14
+// splits) 8.75 / 8.93, 20 of 100-1000 (167 slots a split) 7.23 / 7.49, 4 of
+// 256-2048 6.66 / 6.99.
+static bool shares_by_length(const DecodeArgs& a) {
+  return a.kv_last != nullptr && a.kv_last_sb != 0 && a.bias == nullptr && a.B >= 2 && a.B <= 64 &&
+         a.splits <= 8 && a.cap >= 6 * kTile * a.splits &&
+         (int64_t)(a.cap / kTile + 1) * a.splits * a.B < 0x7fffffff;
+}
+
 template <bool kPaged>
 static void launch_split_paging(const DecodeArgs& a, int mode, hipStream_t st) {
   const dim3 grid(a.splits, a.B * a.KVH);
   const int nw = pick_waves(a, mode);
+  if (mode == kFused && nw <= 8 && shares_by_length(a)) mode = kFusedRows;
   if (nw == 16) launch_nw<16, kPaged>(a, mode, grid, st);
   else if (nw == 8) launch_nw<8, kPaged>(a, mode, grid, st);
   else if (nw == 4) launch_nw<4, kPaged>(a, mode, grid, st);
