@@ -28,10 +28,13 @@ path (``step_ops``, include/qf_step.h): per layer one launch for rms_norm +
 QKV + RoPE + append, the split-K attention launch, one for the split merge +
 o_proj + residual, one for rms_norm + gate/up + SwiGLU and one for down_proj +
 residual; then one for rms_norm + lm_head + per-block argmax and one for the
-argmax and the slot bookkeeping.  5..32 rows run the same step on the wide kernels
-(``wide_ops``, include/qf_wide.h) around the merged attention; larger batches keep the torch
-projections (hipBLASLt / ATen kernels) around the same HIP attention kernels.  Prefill always uses the torch
-projections.  Everything is fp16 storage with the reference's rounding points.
+argmax and the slot bookkeeping.  5..32 rows run the same step on the wide
+kernels (``wide_ops``, include/qf_wide.h) around the merged attention; larger
+batches keep the torch projections (hipBLASLt / ATen kernels) around the same
+HIP attention kernels.  Prefill runs its layers from one native call
+(``prefill_ops``, include/qf_prefill.h) and keeps the torch projections for the
+layouts that call does not take.  Everything is fp16 storage with the
+reference's rounding points.
 """
 
 from __future__ import annotations
