@@ -29,7 +29,9 @@ using step::wave_sum;
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-enum Epilogue { kEpiQkv = 0, kEpiResidual = 1, kEpiSwiglu = 2 };
+// kEpiPartial: fp32 sums of one k share of a residual product, for
+// prefill_rms_kernel to add up.
+enum Epilogue { kEpiQkv = 0, kEpiResidual = 1, kEpiSwiglu = 2, kEpiPartial = 3 };
 
 struct GemmArgs {
   const f16* x;     // (T, K), row stride x_sn
@@ -49,10 +51,9 @@ struct GemmArgs {
   f16* vc;
   int64_t vc_sb, vc_sh, vc_sn;
   int QH, KVH;
-  // split k (residual epilogue)
+  // split k (partial epilogue): (splits, T, N) sums
   int splits;
   float* part;
-  int32_t* ticket;
 };
 
 // 16 bytes per lane from byte `off` of the resource to LDS byte `dst` + 16 *
@@ -92,7 +93,9 @@ template <int kEpi>
 __device__ __forceinline__ void finish(const GemmArgs& a, int f0, int t, int q,
                                        const f32x4 (&acc)[group_blocks(kEpi)]) {
   if (f0 >= a.N) return;
-  if constexpr (kEpi == kEpiResidual) {
+  if constexpr (kEpi == kEpiPartial) {
+    *reinterpret_cast<f32x4*>(a.part + ((int64_t)blockIdx.y * a.T + t) * a.N + f0 + 4 * q) = acc[0];
+  } else if constexpr (kEpi == kEpiResidual) {
     f16* y = a.y + t * a.y_sn + f0 + 4 * q;
     const f16x4 res = *reinterpret_cast<const f16x4*>(y);
     f16x4 o;
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(kWN* kWM* kWK * 64, 1) void prefill_gemm_kernel(Gem
 
   // Stages of this workgroup's k range.
   int s_lo = 0, s_n = K / kBK;
-  if (kEpi == kEpiResidual && a.splits > 1) {
+  if (kEpi == kEpiPartial) {
     const int all = K / kBK;
     s_lo = (int)blockIdx.y * all / a.splits;
     s_n = ((int)blockIdx.y + 1) * all / a.splits - s_lo;
@@ -341,45 +344,6 @@ __global__ __launch_bounds__(kWN* kWM* kWK * 64, 1) void prefill_gemm_kernel(Gem
 #pragma unroll
       for (int s = 1; s < kWK; ++s) g[f] += red[((s * kTW + wk) * kFW + f) * 64 + lane];
     }
-    if (kEpi == kEpiResidual && a.splits > 1) {
-      // Workgroups that share a tile: write-through partials, a ticket per tile,
-      // and the last one sums all of them in split order (the same sum whichever
-      // workgroup is last).  Publication order as in the decode kernel's merge.
-      const int S = a.splits;
-      constexpr int kTileFloats = kBN * kBM;
-      const __amdgpu_buffer_rsrc_t rp =
-          buffer_rsrc(a.part + (int64_t)lin * S * kTileFloats, (int64_t)S * kTileFloats * 4);
-#pragma unroll
-      for (int f = 0; f < kFW; ++f)
-        __builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(u32x4, g[f]), rp,
-            ((int)blockIdx.y * kTileFloats / 4 + (wv * kFW + f) * 64 + lane) * 16, 0, kSc1);
-      s_waitcnt_vm(0);
-      __syncthreads();
-      int* flag = reinterpret_cast<int*>(lds);
-      if (threadIdx.x == 0) *flag = atomicAdd(a.ticket + lin, 1) == S - 1;
-      __syncthreads();
-      if (!*flag) return;
-#pragma unroll
-      for (int f = 0; f < kFW; ++f) g[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < S; s += 2) {
-        f32x4 v[2][kFW];  // a split past S reads zeros: the buffer ends there
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int f = 0; f < kFW; ++f)
-            v[u][f] = __builtin_bit_cast(
-                f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                           rp, ((s + u) * kTileFloats / 4 + (wv * kFW + f) * 64 + lane) * 16, 0,
-                           kSc1));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int f = 0; f < kFW; ++f) g[f] += v[u][f];
-      }
-      if (threadIdx.x == 0) atomicExch(a.ticket + lin, 0);
-    }
     const int tok = tok0 + 16 * wk + r16;
 #pragma unroll
     for (int f = 0; f < kFW; f += GB) {
@@ -392,11 +356,17 @@ __global__ __launch_bounds__(kWN* kWM* kWK * 64, 1) void prefill_gemm_kernel(Gem
 }
 
 // rms_norm of T rows, a row per wave: fp16((x * rsqrt(mean(x^2) + eps)) * w).
+// kParts: first x <- fp16(x + fp16(sum of the row's `splits` partials)), in
+// place and in split order, so a repeat gives the same bits; w == nullptr then
+// ends there.  The whole chip adds the partials up while it would have waited
+// for this row's load anyway; the last workgroup of a tile reading them back
+// (write-through stores, a ticket) was alone with them.
 constexpr int kMaxChunks = 4;  // 16-byte chunks per lane: hidden <= 2048
 
-__global__ __launch_bounds__(256) void prefill_rms_kernel(const f16* __restrict__ x,
-                                                          const f16* __restrict__ w, f16* y, int T,
-                                                          int K, float eps) {
+template <bool kParts>
+__global__ __launch_bounds__(256) void prefill_rms_kernel(f16* x, const f16* __restrict__ w, f16* y,
+                                                          const float* __restrict__ part, int splits,
+                                                          int T, int K, float eps) {
   const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return;
   const int C = K / 8;
@@ -406,8 +376,44 @@ __global__ __launch_bounds__(256) void prefill_rms_kernel(const f16* __restrict_
     if (64 * i < C) {
       const int c = min(64 * i + lane, C - 1);
       v[i] = load16(x + (int64_t)t * K + 8 * c);
-      g[i] = load16(w + 8 * c);
+      if (!kParts || w != nullptr) g[i] = load16(w + 8 * c);
     }
+  if constexpr (kParts) {
+    f32x4 sum[kMaxChunks][2];
+#pragma unroll
+    for (int i = 0; i < kMaxChunks; ++i) sum[i][0] = sum[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < splits; s += 4) {
+      f32x4 p[4][kMaxChunks][2];  // a batch of loads in flight together
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float* row = part + ((int64_t)(s + u) * T + t) * K;
+#pragma unroll
+        for (int i = 0; i < kMaxChunks; ++i) {
+          p[u][i][0] = p[u][i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (64 * i < C && s + u < splits) {
+            const float* src = row + 8 * min(64 * i + lane, C - 1);
+            p[u][i][0] = *reinterpret_cast<const f32x4*>(src);
+            p[u][i][1] = *reinterpret_cast<const f32x4*>(src + 4);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < kMaxChunks; ++i) {
+          sum[i][0] += p[u][i][0];
+          sum[i][1] += p[u][i][1];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kMaxChunks; ++i)
+      if (64 * i + lane < C) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = (f16)((float)v[i][e] + (float)(f16)sum[i][e >> 2][e & 3]);
+        store16(x + (int64_t)t * K + 8 * (64 * i + lane), v[i]);
+      }
+    if (w == nullptr) return;
+  }
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < kMaxChunks; ++i)
@@ -435,10 +441,8 @@ __global__ __launch_bounds__(256) void prefill_tokens_kernel(const int* cu, int 
                                                              const float* inv_freq,
                                                              const int32_t* table, int64_t t_sb,
                                                              int log2p, int ppr, int n_pages,
-                                                             f16* cs, int2* info,
-                                                             int32_t* ticket, int n_tickets) {
+                                                             f16* cs, int2* info) {
   const int t = blockIdx.x * 8 + (threadIdx.x >> 5), i = threadIdx.x & 31;
-  for (int j = blockIdx.x * 256 + threadIdx.x; j < n_tickets; j += gridDim.x * 256) ticket[j] = 0;
   if (t >= T) return;
   int b, pos;
   if (cu != nullptr) {
@@ -514,8 +518,8 @@ static int launch_as(GemmArgs a, hipStream_t st) {
 //   - 128 x 128, half the operand bytes per product of 64 x 64, from nine
 //     tiles per 16 CUs on for gate/up (152 tiles at 256 tokens: 13.8 against
 //     16.1; 608 at 1024: 28.7 against 40.1) and from thirteen for the others
-//     (down at 4096 tokens, 224 tiles: 58.4 against 65.8; at 2048, 112 tiles:
-//     56.8 against 33.8; QKV at 2048, 144 tiles: 17.6 against 17.7);
+//     (down, unsplit, at 4096 tokens, 224 tiles: 58.4 against 65.8; at 2048,
+//     112 tiles: 56.8 against 33.8; QKV at 2048, 144 tiles: 17.6 against 17.7);
 //   - gate/up 160 features wide from two tiles per CU on: its 9728 rows then
 //     fill whole rounds of workgroups (two per CU) at 1024 x n tokens (28.2
 //     against 28.7, at 4096 81.7 against 88.4, at 8192 160 against 199);
@@ -529,13 +533,59 @@ template <int kEpi>
 static int launch(const GemmArgs& a, int cus, hipStream_t st) {
   const int64_t t128 = (int64_t)((a.N + 127) / 128) * ((a.T + 127) / 128);
   const int64_t t64 = (int64_t)((a.N + 63) / 64) * ((a.T + 63) / 64);
-  if (t128 * 16 >= (kEpi == kEpiSwiglu ? 9 : 13) * (int64_t)cus && a.splits == 1) {
+  if (t128 * 16 >= (kEpi == kEpiSwiglu ? 9 : 13) * (int64_t)cus) {
     if constexpr (kEpi == kEpiSwiglu)
       if (t128 >= 2 * (int64_t)cus) return launch_as<10, 2, 1, 4, 1, 64, 2, kEpi>(a, st);
     return launch_as<4, 4, 2, 2, 1, 64, 2, kEpi>(a, st);
   }
-  if (t64 * a.splits <= cus) return launch_as<4, 4, 1, 1, 4, 128, 3, kEpi>(a, st);
+  if (t64 <= cus) return launch_as<4, 4, 1, 1, 4, 128, 3, kEpi>(a, st);
   return launch_as<4, 4, 1, 1, 4, 128, 2, kEpi>(a, st);
+}
+
+// The down projection's k split over workgroups whose partial sums the next
+// rms_norm adds up.
+struct KSplit {
+  int splits;  // 1: not split
+  int form;    // 0: 64 x 64 tiles, 1: 128 x 128 and one workgroup per CU, 2: 128 x 128 and two
+};
+
+// 64 x 64 tiles: as many shares as the CUs hold at one workgroup each, at most
+// eight and none under four stages of 128.
+static int shares64(int T, int N, int K, int cus) {
+  const int tiles = (N + 63) / 64 * ((T + 63) / 64);
+  return std::max(1, std::min({cus / tiles, 8, K / 128 / 4}));
+}
+
+// 128 x 128 tiles: as many shares as the fullest XCD's tiles leave room for in
+// one round of workgroups (of more, the last ones wait for a whole share: 42
+// tiles in 6 shares are 36 workgroups on an XCD's 32 CUs, 2027 us against 1815
+// in 5), none under eight stages of 64.
+static int shares128(int T, int N, int K, int slots) {
+  int most = 0;
+  xcd_split((N + 127) / 128, (T + 127) / 128, (int64_t)T * K * 2, (int64_t)N * K * 2, most);
+  return std::max(1, std::min({slots / 8 / most, 8, K / 64 / 8}));
+}
+
+// Up to one 64 x 64 tile per two CUs the small tiles; then 128 x 128, four
+// stages deep with a CU to itself while that allows two shares, two stages and
+// two workgroups per CU past that.  Measured on MI355X for the whole prefill of
+// 24 layers, us, unsplit or in 64 x 64 shares merged behind a ticket / this
+// rule: 64 tokens 1263 / 1221, 300 1539 / 1495, 512 1792 / 1763; 600 1852 /
+// 1750, 1024 2314 / 2209, 1280 2954 / 2704, 2048 3736 / 3381; 2400 4667 / 4117,
+// 3000 5287 / 4417, 4096 6309 / 5943.  Across the first line: seven 128 x 128
+// shares at 512 tokens 1785, three 64 x 64 ones at 600 1771.
+static KSplit k_split(int T, int N, int K, int cus) {
+  const int64_t t64 = (int64_t)((N + 63) / 64) * ((T + 63) / 64);
+  if (t64 * 2 <= cus) return {shares64(T, N, K, cus), 0};
+  const int one = shares128(T, N, K, cus);
+  if (one > 1) return {one, 1};
+  return {shares128(T, N, K, 2 * cus), 2};
+}
+
+static int launch_split(const GemmArgs& a, int form, hipStream_t st) {
+  if (form == 0) return launch_as<4, 4, 1, 1, 4, 128, 3, kEpiPartial>(a, st);
+  if (form == 1) return launch_as<4, 4, 2, 2, 1, 64, 4, kEpiPartial>(a, st);
+  return launch_as<4, 4, 2, 2, 1, 64, 2, kEpiPartial>(a, st);
 }
 
 }  // namespace pgemm
@@ -546,24 +596,15 @@ using namespace qf::pgemm;
 
 namespace {
 
-// Workgroups sharing a 64 x 64 tile's k in the down projection: as many as the
-// CUs hold at one each, at most eight and none under four stages (4864 wide,
-// us for 1 / 2 / 4 at 64 tokens 16.8 / 12.7 / 10.6, at 256 17.4 / 13.4 / 11.6,
-// for 1 / 2 at 512 18.5 / 14.8).
-int down_splits(int T, int H, int I, int cus) {
-  const int tiles = (H + 63) / 64 * ((T + 63) / 64), stages = I / 128;
-  const int s = std::min({cus / tiles, 8, stages / 4});
-  return s < 1 ? 1 : s;
-}
-
 constexpr int kMaxCus = 256;
 
 struct Workspace {
-  int64_t x, qkv, att, h, cs, info, part, ticket, bytes;
-  int n_tickets, splits;
+  int64_t x, qkv, att, h, cs, info, part, bytes;
 };
 
-Workspace workspace(int T, int H, int QH, int KVH, int I, int cus) {
+// For a whole part's CUs: each form's shares only grow with the CU count, but
+// fewer CUs may take another form, so the partials hold the most of them.
+Workspace workspace(int T, int H, int QH, int KVH, int I) {
   Workspace w;
   int64_t at = 0;
   const auto take = [&](int64_t bytes) {
@@ -577,10 +618,8 @@ Workspace workspace(int T, int H, int QH, int KVH, int I, int cus) {
   w.h = take((int64_t)T * I * 2);
   w.cs = take((int64_t)T * 64 * 2);
   w.info = take((int64_t)T * 8);
-  w.splits = down_splits(T, H, I, cus);
-  w.n_tickets = (H + 63) / 64 * ((T + 63) / 64);
-  w.part = take(w.splits > 1 ? (int64_t)w.n_tickets * w.splits * 64 * 64 * 4 : 0);
-  w.ticket = take((int64_t)w.n_tickets * 4);
+  const int most = std::max(shares64(T, H, I, kMaxCus), shares128(T, H, I, 2 * kMaxCus));
+  w.part = take(most > 1 ? (int64_t)most * T * H * 4 : 0);
   w.bytes = at;
   return w;
 }
@@ -597,8 +636,7 @@ bool shapes_ok(int T, int H, int QH, int KVH, int D, int I) {
 
 extern "C" int64_t qf_prefill_layers_workspace(int T, int hidden, int QH, int KVH, int D, int I) {
   if (!shapes_ok(T, hidden, QH, KVH, D, I)) return QF_ERR_UNSUPPORTED;
-  // The splits, so the bytes, only grow with the CU count: sized for a whole part.
-  return workspace(T, hidden, QH, KVH, I, kMaxCus).bytes;
+  return workspace(T, hidden, QH, KVH, I).bytes;
 }
 
 extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, void* hidden_p, int T,
@@ -613,7 +651,7 @@ extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, voi
   if (!al16(hidden_p) || !al16(ws)) return QF_ERR_INVALID_ARG;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int found = stream_cus(st), cus = found > 0 && found < kMaxCus ? found : kMaxCus;
-  const Workspace w = workspace(T, H, QH, KVH, I, cus);
+  const Workspace w = workspace(T, H, QH, KVH, I);
   if (ws_bytes < w.bytes) return QF_ERR_SCRATCH_LIMIT;
   int l2 = 0;
   if (block_table != nullptr) {
@@ -641,10 +679,19 @@ extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, voi
   f16* cs = reinterpret_cast<f16*>(base + w.cs);
   int2* info = reinterpret_cast<int2*>(base + w.info);
   const int W = (QH + 2 * KVH) * 64, A = QH * 64;
-  const dim3 rms_grid((T + 3) / 4);
+  float* part = reinterpret_cast<float*>(base + w.part);
+  const KSplit down = k_split(T, H, I, cus);
+  const auto norm = [&](const f16* weight, bool parts) {
+    const dim3 grid((T + 3) / 4), block(256);
+    if (parts)
+      hipLaunchKernelGGL(prefill_rms_kernel<true>, grid, block, 0, st, hidden, weight, x, part,
+                         down.splits, T, H, eps);
+    else
+      hipLaunchKernelGGL(prefill_rms_kernel<false>, grid, block, 0, st, hidden, weight, x, nullptr,
+                         0, T, H, eps);
+  };
   hipLaunchKernelGGL(prefill_tokens_kernel, dim3((T + 7) / 8), dim3(256), 0, st, cu, B, S, T,
-                     inv_freq, block_table, bt_sb, l2, pages_per_row, n_pages, cs, info,
-                     reinterpret_cast<int32_t*>(base + w.ticket), w.n_tickets);
+                     inv_freq, block_table, bt_sb, l2, pages_per_row, n_pages, cs, info);
   int rc = (int)hipGetLastError();
   for (int i = 0; i < n_layers && rc == 0; ++i) {
     const QfPrefillLayer& y = layers[i];
@@ -660,11 +707,10 @@ extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, voi
     g.vc = static_cast<f16*>(y.v_cache);
     g.vc_sb = y.vc_sb; g.vc_sh = y.vc_sh; g.vc_sn = y.vc_sn;
     g.bias = static_cast<const f16*>(y.b_qkv);
-    g.part = reinterpret_cast<float*>(base + w.part);
-    g.ticket = reinterpret_cast<int32_t*>(base + w.ticket);
+    g.part = part;
 
-    hipLaunchKernelGGL(prefill_rms_kernel, rms_grid, dim3(256), 0, st, hidden,
-                       static_cast<const f16*>(y.norm1), x, T, H, eps);
+    // Split: the layer before left its down_proj as partials.
+    norm(static_cast<const f16*>(y.norm1), i > 0 && down.splits > 1);
     GemmArgs gq = g;
     gq.x = x; gq.x_sn = H; gq.w = static_cast<const f16*>(y.w_qkv); gq.y = qkv; gq.y_sn = W;
     gq.N = W; gq.K = H;
@@ -685,8 +731,7 @@ extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, voi
     go.N = H; go.K = A;
     rc = launch<kEpiResidual>(go, cus, st);
     if (rc) break;
-    hipLaunchKernelGGL(prefill_rms_kernel, rms_grid, dim3(256), 0, st, hidden,
-                       static_cast<const f16*>(y.norm2), x, T, H, eps);
+    norm(static_cast<const f16*>(y.norm2), false);
     GemmArgs gu = g;
     gu.x = x; gu.x_sn = H; gu.w = static_cast<const f16*>(y.w_gate_up); gu.y = h; gu.y_sn = I;
     gu.N = 2 * I; gu.K = H;
@@ -695,8 +740,12 @@ extern "C" int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, voi
     GemmArgs gd = g;
     gd.x = h; gd.x_sn = I; gd.w = static_cast<const f16*>(y.w_down); gd.y = hidden; gd.y_sn = H;
     gd.N = H; gd.K = I;
-    gd.splits = w.splits;
-    rc = launch<kEpiResidual>(gd, cus, st);
+    gd.splits = down.splits;
+    rc = down.splits > 1 ? launch_split(gd, down.form, st) : launch<kEpiResidual>(gd, cus, st);
+  }
+  if (rc == 0 && down.splits > 1) {
+    norm(nullptr, true);
+    rc = (int)hipGetLastError();
   }
   return rc;
 }

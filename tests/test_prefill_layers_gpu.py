@@ -52,6 +52,7 @@ def _native_only(engine):
 
 @pytest.mark.parametrize("lengths", [
     (1,), (63,), (64,), (65,), (127,), (128,), (129,), (300,), (1025,), (2048,), (2113,),
+    (512,), (513,), (577,), (1281,), (2305,), (3585,), (4608,), (4609,),
     (5, 5, 5), (128, 128), (700, 700, 700),
     (3, 70, 1, 64), (257, 31, 900), (0, 40, 0, 65, 0),
 ])
@@ -97,8 +98,8 @@ def test_prefill_paged_matches_torch_projections(dev, weights, lengths, page):
 
 
 def test_graph_replays_equal_eager(dev, weights):
-    """Captured with the split down projection, replayed on changed inputs: the
-    tickets are cleared by the call itself, the result is the eager one's bits."""
+    """Captured with the split down projection, replayed on changed inputs:
+    the result is the eager one's bits."""
     eng = DecodeEngine(CFG, weights, dev)
     caches = eng.new_caches(1, 64)
     embed = weights["embed"]
