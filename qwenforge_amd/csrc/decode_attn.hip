@@ -151,9 +151,9 @@ __device__ __forceinline__ int lane_scan(int v) {
 // < B <= 64 works out row r.  Returns false for a spare workgroup.
 constexpr int kMaxRowSplits = 16;
 struct RowShare {
-  int b, s, splits, span, base;
+  int b, s, splits, span, base;  // base: scratch slot of the row's first partial
 };
-__device__ __forceinline__ bool row_share(const DecodeArgs& a, int u, RowShare& r) {
+__device__ __forceinline__ bool row_share(const DecodeArgs& a, int h, int u, RowShare& r) {
   const int lane = threadIdx.x & 63;
   const int64_t last = a.kv_last[(int64_t)min(lane, a.B - 1) * a.kv_last_sb];
   const int span = lane < a.B ? valid_slots(a, last) : 0;
@@ -166,9 +166,10 @@ __device__ __forceinline__ bool row_share(const DecodeArgs& a, int u, RowShare& 
   const int row = __builtin_popcountll(__ballot(lane < a.B && end - n <= u)) - 1;
   r.b = row;
   r.splits = __builtin_amdgcn_readlane(n, row);
-  r.base = __builtin_amdgcn_readlane(end, row) - r.splits;
+  const int first = __builtin_amdgcn_readlane(end, row) - r.splits;
+  r.base = h * a.splits * a.B + first;
   r.span = __builtin_amdgcn_readlane(span, row);
-  r.s = u - r.base;
+  r.s = u - first;
   return r.s < r.splits;
 }
 
@@ -211,9 +212,9 @@ __device__ __forceinline__ void lse_merge_lanes(float& M, float& L, f32x4& A) {
   A = a0;
 }
 
-// Folds the S partials of query q of one (b, h), the first in scratch slot
-// pbase, into the running state (M, L, A)
-// of dims 4*d4 .. +3, d4 = lane % 16.  The wave's four 16-lane rows hold the
+// Folds the partials of query q of (b, h) = bh -- `splits` from scratch slot
+// bh * splits on; kRows: the share's, from its base on -- into the running
+// state (M, L, A) of dims 4*d4 .. +3, d4 = lane % 16.  The wave's four 16-lane rows hold the
 // consecutive subs sub0 + lane / 16 out of nsub; sub folds partials
 // j = sub + nsub * u, batch after batch of kB (j < S).  In a batch the wave
 // loads each of its 4 kB partials' (m, l) once -- lane i loads partial
@@ -229,13 +230,15 @@ __device__ __forceinline__ void lse_merge_lanes(float& M, float& L, f32x4& A) {
 // instead of a read of whatever follows the scratch.
 // kCoherent: sc1 loads, for partials that other workgroups of the same
 // launch stored with sc1 stores.
-template <int kB, bool kCoherent>
-__device__ __forceinline__ void fold_wave(const DecodeArgs& a, int64_t pbase, int S, int q, int lane,
-                                          int sub0, int nsub, float& M, float& L, f32x4& A) {
+template <int kB, bool kCoherent, bool kRows>
+__device__ __forceinline__ void fold_wave(const DecodeArgs& a, int bh, const RowShare& r, int q,
+                                          int lane, int sub0, int nsub, float& M, float& L,
+                                          f32x4& A) {
   static_assert(4 * kB <= 64, "a batch's (m, l) must fit one load per lane");
-  const int G = a.G;
+  const int G = a.G, S = kRows ? r.splits : a.splits;
   const int s4 = lane >> 4, d4 = lane & 15, sub = sub0 + s4;
   constexpr int aux = kCoherent ? kSc1 : 0;
+  const int64_t pbase = kRows ? r.base : (int64_t)bh * S;
   const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(a.acc + pbase * G * kD, (int64_t)S * G * kD * 4);
   const __amdgpu_buffer_rsrc_t rm = buffer_rsrc(a.m + pbase * G, (int64_t)S * G * 4);
   const __amdgpu_buffer_rsrc_t rl = buffer_rsrc(a.l + pbase * G, (int64_t)S * G * 4);
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
   const int h = bh % KVH;
   RowShare share = {0, 0, 0, 0, 0};
   if constexpr (kMode == kFusedRows) {
-    if (!row_share(a, b * a.splits + s, share)) return;
+    if (!row_share(a, h, b * a.splits + s, share)) return;
     b = share.b;
     s = share.s;
     bh = b * KVH + h;
@@ -608,9 +611,7 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
 
   constexpr bool kRows = kMode == kFusedRows;
   const int S = kRows ? share.splits : a.splits, G = a.G;
-  const int64_t pbase =
-      kRows ? (int64_t)h * a.splits * a.B + share.base : (int64_t)bh * a.splits;
-  const int64_t part = pbase + s;
+  const int64_t part = kRows ? share.base + s : (int64_t)bh * S + s;
   if (w < 4) {
     float mw[NW], wt[NW];
     float M = kNegInf;
@@ -680,8 +681,8 @@ __global__ __launch_bounds__(NW * 64) void decode_split_kernel(DecodeArgs a) {
     for (int q = w; q < G; q += NW) {
       float Mq = kNegInf, Lq = 0.f;
       f32x4 Aq = {0.f, 0.f, 0.f, 0.f};
-      if (S <= 16) fold_wave<4, true>(a, pbase, S, q, lane, 0, 4, Mq, Lq, Aq);
-      else fold_wave<8, true>(a, pbase, S, q, lane, 0, 4, Mq, Lq, Aq);
+      if (S <= 16) fold_wave<4, true, kRows>(a, bh, share, q, lane, 0, 4, Mq, Lq, Aq);
+      else fold_wave<8, true, kRows>(a, bh, share, q, lane, 0, 4, Mq, Lq, Aq);
       lse_merge_lanes<false>(Mq, Lq, Aq);
       lse_merge_lanes<true>(Mq, Lq, Aq);
       if (lane < 16) store_out(a, bh, q, lane, Lq, Aq);
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a) {
   const int d4 = lane & 15;
   float M = kNegInf, L = 0.f;
   f32x4 A = {0.f, 0.f, 0.f, 0.f};
-  fold_wave<8, false>(a, (int64_t)bh * a.splits, a.splits, q, lane, 4 * w, 16, M, L, A);
+  fold_wave<8, false, false>(a, bh, {}, q, lane, 4 * w, 16, M, L, A);
   lse_merge_lanes<false>(M, L, A);
   lse_merge_lanes<true>(M, L, A);
   if (w > 0 && lane < 16) {
