@@ -85,18 +85,13 @@ int qf_abi_version(void);
  *          With splits = 1 one workgroup per (b, kv head) covers every slot,
  *          merges its waves in LDS and writes `out` itself: acc, m, l and the
  *          ticket are not read or written.
- *          With a ticket, kv_last per row, no bias, splits <= 8 and
- *          cap >= 192 * splits the B * splits workgroups of a kv head are
- *          shared out by the rows' lengths instead (up to 16 splits for a
- *          long row), so a row's rounding then depends on the other rows'
- *          bounds too; the partials of one kv head lie together.
  *   ticket NULL: the merge runs as a second kernel (reference two-launch
  *          shape).  Non-NULL: int32[B*KVH], one counter per (b, kv head),
  *          zero-filled once by the caller; the merge runs inside the same
  *          launch: every workgroup of a (b, h) stores its partial, waits for
  *          the stores to complete and increments the counter, and the
- *          workgroup that completes the count (one increment a split) merges all
- *          partials of the row, writes the output and re-arms the counter to 0,
+ *          workgroup that completes the count (splits increments) merges all
+ *          `splits` partials, writes the output and re-arms the counter to 0,
  *          so the same ticket serves every later call.  Calls that share a
  *          ticket or the partials must not overlap in time.
  *   out    (B, KVH, G, D) fp16, strides o_sb, o_sh, o_sg.
@@ -112,6 +107,26 @@ int qf_decode_attn(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
                    void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
                    int B, int KVH, int G, int D, int cap, float scale,
                    void* stream);
+
+/*
+ * qf_decode_attn that may share its workgroups out by the rows' lengths: with
+ * a ticket, 2..64 rows with a kv_last each, no bias, 2..8 splits and
+ * cap >= 192 * splits, the B * splits workgroups of a kv head go to the rows
+ * in proportion to their valid slots (one at least, 16 at most each) instead of
+ * `splits` to every row.  A row's rounding then depends on the other rows'
+ * bounds too, and acc, m and l are scratch without a layout of their own.  Any
+ * other call is qf_decode_attn's, bit for bit.
+ */
+int qf_decode_attn_shared(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                          const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                          const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                          const void* bias, int64_t bias_sb,
+                          const int64_t* kv_last, int64_t kv_last_sb,
+                          float* acc, float* m, float* l, int splits,
+                          int32_t* ticket,
+                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
+                          int B, int KVH, int G, int D, int cap, float scale,
+                          void* stream);
 
 /*
  * Launch plan of the decode split kernel (host only, no GPU work): the

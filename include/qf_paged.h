@@ -59,6 +59,19 @@ int qf_decode_attn_paged(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg
                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
                          int B, int KVH, int G, int D, float scale, void* stream);
 
+/* qf_decode_attn_shared (qf_attn.h) over paged caches. */
+int qf_decode_attn_paged_shared(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                                const void* k_pool, int64_t kp_sp, int64_t kp_sh, int64_t kp_sn,
+                                const void* v_pool, int64_t vp_sp, int64_t vp_sh, int64_t vp_sn,
+                                const int32_t* block_table, int64_t bt_sb, int pages_per_row,
+                                int n_pages, int page_size,
+                                const void* bias, int64_t bias_sb,
+                                const int64_t* kv_last, int64_t kv_last_sb,
+                                float* acc, float* m, float* l, int splits,
+                                int32_t* ticket,
+                                void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
+                                int B, int KVH, int G, int D, float scale, void* stream);
+
 /*
  * Split phase only, over paged caches (qf_decode_split semantics, the
  * _flash_decode_split_kernel launch SE:854-865): writes the partials

@@ -282,6 +282,10 @@ SIGNATURES = {
     "qf_abi_version": [],
 }
 
+# The same arguments as the calls that give every row the same splits.
+for _name in ("qf_decode_attn", "qf_decode_attn_paged"):
+    SIGNATURES[_name + "_shared"] = SIGNATURES[_name]
+
 # Entry points that do not return an int status.
 RESTYPES = {"qf_error_string": C.c_char_p, "qf_prefill_layers_workspace": _i64}
 

@@ -792,6 +792,7 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // first's compute (config 3, 8 tiles per split: 4 waves 10.57 us, 8 waves
 // 10.80).
 static int pick_waves(const DecodeArgs& a, int mode) {
+  if (mode == kFusedRows) mode = kFused;
   const int64_t wgs = (int64_t)a.splits * a.B * a.KVH;
   int nw = wgs <= 2 ? 16 : (wgs <= 512 ? 8 : 4);
   const int split_len = (a.cap + a.splits - 1) / a.splits;
@@ -854,9 +855,10 @@ static int make_args(DecodeArgs& a, const void* q, int64_t q_sb, int64_t q_sh, i
 }
 
 
-// Whether a single-launch merge shares its workgroups out by the rows' lengths:
-// rows with bounds of their own (and no bias, which may mask anything), at most
-// eight splits a row and at least six tiles of capacity for each.  Measured on
+// Whether a single-launch merge that may share its workgroups out by the rows'
+// lengths does: rows with bounds of their own (and no bias, which may mask
+// anything), at most eight splits a row and at least six tiles of capacity for
+// each (up to eight waves: more are for grids of two workgroups).  Measured on
 // MI355X, us per call, even / shared: paged 16 rows of 201-6007 slots 12.45 /
 // 10.42, 24 of 50-2800 10.59 / 9.50, 32 of 50-2000 10.52 / 9.24, equal rows
 // 13.84 / 13.94 (16 of 6000) and 11.46 / 11.31 (32 of 2000).  Outside the rule
@@ -866,14 +868,13 @@ static int make_args(DecodeArgs& a, const void* q, int64_t q_sb, int64_t q_sh, i
 static bool shares_by_length(const DecodeArgs& a) {
   return a.kv_last != nullptr && a.kv_last_sb != 0 && a.bias == nullptr && a.B >= 2 && a.B <= 64 &&
          a.splits <= 8 && a.cap >= 6 * kTile * a.splits &&
-         (int64_t)(a.cap / kTile + 1) * a.splits * a.B < 0x7fffffff;
+         (int64_t)(a.cap / kTile + 1) * a.splits * a.B < 0x7fffffff && pick_waves(a, kFused) <= 8;
 }
 
 template <bool kPaged>
 static void launch_split_paging(const DecodeArgs& a, int mode, hipStream_t st) {
   const dim3 grid(a.splits, a.B * a.KVH);
   const int nw = pick_waves(a, mode);
-  if (mode == kFused && nw <= 8 && shares_by_length(a)) mode = kFusedRows;
   if (nw == 16) launch_nw<16, kPaged>(a, mode, grid, st);
   else if (nw == 8) launch_nw<8, kPaged>(a, mode, grid, st);
   else if (nw == 4) launch_nw<4, kPaged>(a, mode, grid, st);
@@ -889,6 +890,30 @@ static void launch_combine(const DecodeArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(decode_combine_kernel, dim3(a.B * a.KVH * a.G), dim3(256), 0, st, a);
 }
 
+// Split and merge; `share`: workgroups may be shared out by the rows' lengths.
+static int launch_attn(const DecodeArgs& a, bool share, hipStream_t st) {
+  int mode = merge_mode(a.splits, a.ticket != nullptr);
+  if (share && mode == kFused && shares_by_length(a)) mode = kFusedRows;
+  launch_split_mode(a, mode, st);
+  if (mode == kPartial) launch_combine(a, st);
+  return (int)hipGetLastError();
+}
+
+static int decode_attn(bool share, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn, const void* v,
+                       int64_t v_sb, int64_t v_sh, int64_t v_sn, const void* bias, int64_t bias_sb,
+                       const int64_t* kv_last, int64_t kv_last_sb, float* acc, float* m, float* l,
+                       int splits, int32_t* ticket, void* out, int64_t o_sb, int64_t o_sh,
+                       int64_t o_sg, int B, int KVH, int G, int D, int cap, float scale,
+                       void* stream) {
+  DecodeArgs a;
+  const int rc = make_args(a, q, q_sb, q_sh, q_sg, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn,
+                           bias, bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out,
+                           o_sb, o_sh, o_sg, B, KVH, G, D, cap, scale, true, true);
+  if (rc != QF_OK) return rc;
+  return launch_attn(a, share, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int qf_decode_attn(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
                               const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                               const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -899,16 +924,24 @@ extern "C" int qf_decode_attn(const void* q, int64_t q_sb, int64_t q_sh, int64_t
                               void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
                               int B, int KVH, int G, int D, int cap, float scale,
                               void* stream) {
-  DecodeArgs a;
-  const int rc = make_args(a, q, q_sb, q_sh, q_sg, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn,
-                           bias, bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out,
-                           o_sb, o_sh, o_sg, B, KVH, G, D, cap, scale, true, true);
-  if (rc != QF_OK) return rc;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int mode = merge_mode(splits, ticket != nullptr);
-  launch_split_mode(a, mode, st);
-  if (mode == kPartial) launch_combine(a, st);
-  return (int)hipGetLastError();
+  return decode_attn(false, q, q_sb, q_sh, q_sg, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, bias,
+                     bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb, o_sh, o_sg,
+                     B, KVH, G, D, cap, scale, stream);
+}
+
+extern "C" int qf_decode_attn_shared(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                                     const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                                     const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                                     const void* bias, int64_t bias_sb,
+                                     const int64_t* kv_last, int64_t kv_last_sb,
+                                     float* acc, float* m, float* l, int splits,
+                                     int32_t* ticket,
+                                     void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
+                                     int B, int KVH, int G, int D, int cap, float scale,
+                                     void* stream) {
+  return decode_attn(true, q, q_sb, q_sh, q_sg, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, bias,
+                     bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb, o_sh, o_sg,
+                     B, KVH, G, D, cap, scale, stream);
 }
 
 extern "C" int qf_decode_waves(int B, int KVH, int G, int cap, int splits, int fused) {
@@ -987,6 +1020,26 @@ static int make_paged(DecodeArgs& a, int64_t kp_sp, int64_t vp_sp, const int32_t
   return QF_OK;
 }
 
+static int decode_attn_paged(bool share, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                             const void* k_pool, int64_t kp_sp, int64_t kp_sh, int64_t kp_sn,
+                             const void* v_pool, int64_t vp_sp, int64_t vp_sh, int64_t vp_sn,
+                             const int32_t* block_table, int64_t bt_sb, int pages_per_row,
+                             int n_pages, int page_size, const void* bias, int64_t bias_sb,
+                             const int64_t* kv_last, int64_t kv_last_sb, float* acc, float* m,
+                             float* l, int splits, int32_t* ticket, void* out, int64_t o_sb,
+                             int64_t o_sh, int64_t o_sg, int B, int KVH, int G, int D, float scale,
+                             void* stream) {
+  if (page_log2(page_size, pages_per_row, n_pages) < 0) return QF_ERR_UNSUPPORTED;
+  DecodeArgs a;
+  int rc = make_args(a, q, q_sb, q_sh, q_sg, k_pool, 0, kp_sh, kp_sn, v_pool, 0, vp_sh, vp_sn,
+                     bias, bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb,
+                     o_sh, o_sg, B, KVH, G, D, pages_per_row * page_size, scale, true, true);
+  if (rc == QF_OK)
+    rc = make_paged(a, kp_sp, vp_sp, block_table, bt_sb, pages_per_row, n_pages, page_size);
+  if (rc != QF_OK) return rc;
+  return launch_attn(a, share, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int qf_decode_attn_paged(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
                                     const void* k_pool, int64_t kp_sp, int64_t kp_sh, int64_t kp_sn,
                                     const void* v_pool, int64_t vp_sp, int64_t vp_sh, int64_t vp_sn,
@@ -998,19 +1051,27 @@ extern "C" int qf_decode_attn_paged(const void* q, int64_t q_sb, int64_t q_sh, i
                                     int32_t* ticket,
                                     void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
                                     int B, int KVH, int G, int D, float scale, void* stream) {
-  if (page_log2(page_size, pages_per_row, n_pages) < 0) return QF_ERR_UNSUPPORTED;
-  DecodeArgs a;
-  int rc = make_args(a, q, q_sb, q_sh, q_sg, k_pool, 0, kp_sh, kp_sn, v_pool, 0, vp_sh, vp_sn,
-                     bias, bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb,
-                     o_sh, o_sg, B, KVH, G, D, pages_per_row * page_size, scale, true, true);
-  if (rc == QF_OK)
-    rc = make_paged(a, kp_sp, vp_sp, block_table, bt_sb, pages_per_row, n_pages, page_size);
-  if (rc != QF_OK) return rc;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int mode = merge_mode(splits, ticket != nullptr);
-  launch_split_mode(a, mode, st);
-  if (mode == kPartial) launch_combine(a, st);
-  return (int)hipGetLastError();
+  return decode_attn_paged(false, q, q_sb, q_sh, q_sg, k_pool, kp_sp, kp_sh, kp_sn, v_pool, vp_sp, vp_sh,
+                           vp_sn, block_table, bt_sb, pages_per_row, n_pages, page_size, bias,
+                           bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb, o_sh,
+                           o_sg, B, KVH, G, D, scale, stream);
+}
+
+extern "C" int qf_decode_attn_paged_shared(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
+                                           const void* k_pool, int64_t kp_sp, int64_t kp_sh, int64_t kp_sn,
+                                           const void* v_pool, int64_t vp_sp, int64_t vp_sh, int64_t vp_sn,
+                                           const int32_t* block_table, int64_t bt_sb, int pages_per_row,
+                                           int n_pages, int page_size,
+                                           const void* bias, int64_t bias_sb,
+                                           const int64_t* kv_last, int64_t kv_last_sb,
+                                           float* acc, float* m, float* l, int splits,
+                                           int32_t* ticket,
+                                           void* out, int64_t o_sb, int64_t o_sh, int64_t o_sg,
+                                           int B, int KVH, int G, int D, float scale, void* stream) {
+  return decode_attn_paged(true, q, q_sb, q_sh, q_sg, k_pool, kp_sp, kp_sh, kp_sn, v_pool, vp_sp, vp_sh,
+                           vp_sn, block_table, bt_sb, pages_per_row, n_pages, page_size, bias,
+                           bias_sb, kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb, o_sh,
+                           o_sg, B, KVH, G, D, scale, stream);
 }
 
 extern "C" int qf_decode_split_paged(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
@@ -1137,9 +1198,7 @@ extern "C" int qf_decode_attn_noalloc(const void* q, int64_t q_sb, int64_t q_sh,
                  kv_last, kv_last_sb, acc, m, l, splits, ticket, out, o_sb, o_sh, o_sg, B, KVH,
                  G, D, cap, scale, true, true);
   if (rc != QF_OK) return rc;
-  launch_split_mode(a, mode, st);
-  if (mode == kPartial) launch_combine(a, st);
-  return (int)hipGetLastError();
+  return launch_attn(a, false, st);
 }
 
 #endif  // QF_DECODE_FUSED_VEC_UNIT

@@ -284,7 +284,7 @@ def _qkv_bias_args(grouped, key_cache, value_cache, attn_bias, kv_last, kv_last_
 def flash_decode_attention(grouped: torch.Tensor, key_cache: torch.Tensor,
                            value_cache: torch.Tensor, attn_bias: torch.Tensor | None,
                            flash, kv_last: torch.Tensor | None = None,
-                           scale: float | None = None) -> torch.Tensor:
+                           scale: float | None = None, share_rows: bool = True) -> torch.Tensor:
     """Drop-in for ``StudentEngine._flash_decode_attention`` (SE:834-874).
 
     grouped (B, KVH, G, D) fp16; key_cache/value_cache (B, KVH, cap, D) fp16;
@@ -295,20 +295,26 @@ def flash_decode_attention(grouped: torch.Tensor, key_cache: torch.Tensor,
     merge.  ``kv_last`` (optional, device int64, shape (1,) or (B,)) is the
     last slot that can be valid; slots after it are skipped (the engine passes
     its ``write_index``).  Writes and returns ``out``.
+
+    ``share_rows``: rows with a ``kv_last`` each may share the call's
+    workgroups out by their lengths (``qf_decode_attn_shared``), faster on
+    ragged batches, and a row's last bits then depend on the other rows'
+    lengths; the partials in ``flash[:3]`` have no layout of their own.  False:
+    every row gets ``acc.shape[2]`` splits whatever the others hold.
     """
     acc, m, l, out, ticket, splits, cap, kv_last_sb = _decode_args(
         grouped, key_cache, value_cache, attn_bias, flash, kv_last)
     b, kvh, g, d = grouped.shape
     scale = d ** -0.5 if scale is None else scale
-    lib = _lib.load()
+    name = "qf_decode_attn_shared" if share_rows else "qf_decode_attn"
     with torch.cuda.device(grouped.device):
-        rc = lib.qf_decode_attn(
+        rc = getattr(_lib.load(), name)(
             *_qkv_bias_args(grouped, key_cache, value_cache, attn_bias, kv_last, kv_last_sb),
             acc.data_ptr(), m.data_ptr(), l.data_ptr(), splits,
             _ptr(ticket),
             out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
             b, kvh, g, d, cap, float(scale), _stream(grouped.device))
-    _lib.check(rc, "qf_decode_attn")
+    _lib.check(rc, name)
     return out
 
 

@@ -162,25 +162,27 @@ def _paged_decode_args(grouped, k_pool, v_pool, block_table, attn_bias, flash, k
 
 def flash_decode_attention_paged(grouped: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
                                  block_table: torch.Tensor, attn_bias: torch.Tensor | None, flash,
-                                 kv_last: torch.Tensor | None = None,
-                                 scale: float | None = None) -> torch.Tensor:
+                                 kv_last: torch.Tensor | None = None, scale: float | None = None,
+                                 share_rows: bool = True) -> torch.Tensor:
     """``flash_decode_attention`` over paged caches (SE:834-874 semantics).
 
     grouped (B, KVH, G, 64); pools (n_pages, KVH, P, 64); block_table
     (B, pages_per_row) int32; attn_bias (B, pages_per_row * P) or None;
     ``flash`` as in ``ops.make_flash_scratch``; kv_last (1,) or (B,) int64
-    bounds each row's slots.  Writes and returns ``flash[3]``.
+    bounds each row's slots; ``share_rows`` as in
+    ``ops.flash_decode_attention``.  Writes and returns ``flash[3]``.
     """
     head, pool, bias, acc, m, l, out, ticket, splits = _paged_decode_args(
         grouped, k_pool, v_pool, block_table, attn_bias, flash, kv_last)
     b, kvh, g, d = grouped.shape
     scale = d ** -0.5 if scale is None else scale
+    name = "qf_decode_attn_paged_shared" if share_rows else "qf_decode_attn_paged"
     with torch.cuda.device(grouped.device):
-        rc = _lib.load().qf_decode_attn_paged(
+        rc = getattr(_lib.load(), name)(
             *head, *pool, *bias, acc.data_ptr(), m.data_ptr(), l.data_ptr(), splits, _ptr(ticket),
             out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
             b, kvh, g, d, float(scale), _stream(grouped.device))
-    _lib.check(rc, "qf_decode_attn_paged")
+    _lib.check(rc, name)
     return out
 
 

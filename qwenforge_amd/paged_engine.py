@@ -68,11 +68,15 @@ class PagedDecodeEngine(DecodeEngine):
                 page_size=kv.page_size))
 
     # ------------------------------------------------------------------ decode
-    def make_paged_context(self, kv: paged.PagedKvCache, batch: int, n_cols: int):
+    def make_paged_context(self, kv: paged.PagedKvCache, batch: int, n_cols: int,
+                           share_rows: bool = False):
         """Static buffers of the paged graph step over rows [0, batch) of ``kv``.
 
         ``pos[b]`` is row b's next slot (= its length so far) and its position;
-        ``rows[:, step]`` receives each replay's tokens (``n_cols`` columns)."""
+        ``rows[:, step]`` receives each replay's tokens (``n_cols`` columns).
+        ``share_rows``: attention may share its workgroups out by the rows'
+        lengths (``ops.flash_decode_attention``); without it a row's results do
+        not depend on the other rows."""
         cfg = self.cfg
         dev = self.device
         fused = self.uses_fused_step(batch)
@@ -94,6 +98,7 @@ class PagedDecodeEngine(DecodeEngine):
             "logits": torch.zeros(batch, cfg.vocab, device=dev, dtype=torch.float16),
             "fused": fused,
             "wide": self.uses_wide_step(batch),
+            "share_rows": share_rows,
         }
         self._step_buffers(ctx, batch)
         return ctx
@@ -147,7 +152,8 @@ class PagedDecodeEngine(DecodeEngine):
 
         def attend(i, grouped):
             return paged.flash_decode_attention_paged(grouped, *kv.pools[i], table, None,
-                                                      ctx["flash"], kv_last=pos, scale=self.scale)
+                                                      ctx["flash"], kv_last=pos, scale=self.scale,
+                                                      share_rows=ctx["share_rows"])
 
         self._wide_body(ctx, qkv, attend, None)
 
@@ -163,7 +169,8 @@ class PagedDecodeEngine(DecodeEngine):
             q_rot = paged.rope_append_paged(q, k, v, cos, sin, kp, vp, table, pos)
             grouped = q_rot.view(b, cfg.kv_heads, cfg.groups, cfg.head_dim)
             att = paged.flash_decode_attention_paged(grouped, kp, vp, table, None, ctx["flash"],
-                                                     kv_last=pos, scale=self.scale)
+                                                     kv_last=pos, scale=self.scale,
+                                                     share_rows=ctx["share_rows"])
             hidden = residual + F.linear(att.reshape(b, 1, cfg.hidden), layer["o_weight"])
             residual = hidden
             hidden = residual + self._mlp(self._rms(hidden, layer["post_norm"]), layer)
@@ -217,7 +224,7 @@ class PagedDecodeEngine(DecodeEngine):
         ev[0].record()
         first = torch.argmax(self.prefill_paged(prompts, kv, range(b)), dim=-1)
         ev[1].record()
-        ctx = self.make_paged_context(kv, b, max_new_tokens)
+        ctx = self.make_paged_context(kv, b, max_new_tokens, share_rows=True)
         self.capture_paged(ctx)
         ctx["rows"][:, 0] = first
         ctx["token"].copy_(first)
@@ -246,8 +253,9 @@ class PagedDecodeEngine(DecodeEngine):
         requests finish, their pages return to the pool and the next waiting
         requests (first come, first served) are prefilled, each on its own, into
         the freed rows; the graph then keeps replaying.  A request's tokens do
-        not depend on the requests it shares the batch with.  A row with no
-        request is parked at slot -1: it appends nothing and its output is
+        not depend on the requests it shares the batch with, for one shape of
+        the step: ``max_batch`` rows of the pages that the longest request
+        needs.  A row with no request is parked at slot -1: it appends nothing and its output is
         ignored.  Returns a list of 1-D id tensors, one per prompt.
         """
         n_req = len(prompts)
@@ -291,7 +299,8 @@ class PagedDecodeEngine(DecodeEngine):
             rows = [r for r, _ in batch]
             # One prefill per request: its projections then have the same
             # shapes whatever it is admitted with, so its tokens do not depend
-            # on the other rows (the decode step is row-independent too).
+            # on the other rows (the decode step is row-independent too: its
+            # context shares no workgroups between rows).
             first = torch.cat([torch.argmax(self.prefill_paged([prompts[i]], kv, [r]), dim=-1)
                                for r, i in batch])
             idx = torch.tensor(rows, device=self.device)

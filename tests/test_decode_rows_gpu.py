@@ -92,3 +92,21 @@ def test_graph_replays_follow_moving_bounds(dev):
         graph.replay()
         _check(flash[3], q, k, v, rows)
         torch.cuda.synchronize()
+
+
+def test_even_splits_on_request(dev):
+    """``share_rows=False``: the reference's partials per row (the combine
+    launch merges them to the same output) and no trace of the other rows."""
+    lengths, cap = [1, 900, 1600, 40, 1599], 1600
+    q, k, v, last = _case(dev, lengths, cap, 7, 3)
+    flash = ops.make_flash_scratch(5, KVH, 7, cap, dev, splits=8, fused=True)
+    print("[decode rows] even", flush=True)
+    first = ops.flash_decode_attention(q, k, v, None, flash, kv_last=last, share_rows=False).clone()
+    _check(first, q, k, v, lengths)
+    merged = ops.flash_decode_combine(flash[:4])
+    assert (merged.float() - first.float()).abs().max().item() <= TOL
+    for others in (0, 300, 1599):
+        moved = torch.full_like(last, others)
+        moved[1] = last[1]
+        out = ops.flash_decode_attention(q, k, v, None, flash, kv_last=moved, share_rows=False)
+        assert torch.equal(out[1], first[1])

@@ -110,3 +110,47 @@ def test_generate_paged_shapes_and_pages(dev):
     assert rows.shape == (3, 12)
     # Pages: ceil((len + 11) / 64) per row.
     assert timing["pages"] == 5 + 1 + 17
+
+
+@pytest.mark.parametrize("batch", [5, 15, 16, 32])
+def test_rows_keep_their_bits_in_any_company(dev, batch):
+    """The paged step over 1600 slots a row (from 15 rows on the attention
+    could share its workgroups out by length): one row's logits, bit for bit,
+    with the other rows parked, short, or full."""
+    cfg = Qwen2Config(layers=2, vocab=4096)
+    eng = PagedDecodeEngine(cfg, init_weights(cfg, dev, seed=9), dev)
+    kv = eng.new_paged_cache(batch, 25 * batch, 64, 25)
+    gen = torch.Generator(dev).manual_seed(1)
+    for pool in (t for pair in kv.pools for t in pair):
+        pool.normal_(generator=gen)
+    for r in range(batch):
+        kv.map_row(r, 1600)
+    ctx = eng.make_paged_context(kv, batch, 4)
+    eng.capture_paged(ctx)
+    print(f"[paged company] B={batch}", flush=True)
+    seen = []
+    for others in (-1, 70, 1590):
+        ctx["pos"].fill_(others)
+        ctx["pos"][1] = 1100
+        ctx["token"].fill_(17)
+        ctx["step"].fill_(0)
+        ctx["graph"].replay()
+        seen.append(ctx["logits"][1].clone())
+    assert torch.equal(seen[0], seen[1]) and torch.equal(seen[0], seen[2])
+
+
+def test_continuous_batching_at_sixteen_rows(dev):
+    """Served among fifteen others at 1536 slots a row, or beside the longest
+    request alone (the same step shape): the same tokens."""
+    cfg = Qwen2Config(layers=2)
+    eng = PagedDecodeEngine(cfg, init_weights(cfg, dev, seed=7), dev)
+    gen = torch.Generator().manual_seed(3)
+    lengths = [1500] + [40 + 90 * i for i in range(16)]
+    prompts = [torch.randint(0, cfg.vocab, (n,), generator=gen).to(dev) for n in lengths]
+    news = [6 + i % 5 for i in range(17)]
+    print("[serve] max_batch=16", flush=True)
+    got = eng.serve(prompts, news, max_batch=16)
+    assert eng._ctx["kv"].capacity == 1536 and eng._ctx["wide"]
+    for i in (0, 3, 9, 16):
+        alone = eng.serve([prompts[i], prompts[0]], [news[i], news[0]], max_batch=16)[0]
+        assert torch.equal(got[i].cpu(), alone.cpu()), f"request {i}"
