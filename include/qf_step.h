@@ -135,7 +135,8 @@ int qf_rms_lm_head(const void* x, int64_t x_sb, const void* norm_w, float eps,
 /* Reduces the per-block keys of qf_rms_lm_head to the argmax token and does
  * the step's slot bookkeeping on the device: token[b] = argmax;
  * rows[b * rows_sb + step[0]] = token[b] (when step[0] < n_rows); then
- * write_index[0] += 1, pos[b] += 1 and step[0] += 1.  Replaces the argmax of
+ * write_index[0] += 1, pos[b] += 1 (a negative one, a parked row's, stays)
+ * and step[0] += 1.  Replaces the argmax of
  * :982 and the host-side updates between replays (student_engine.py:1126-1132:
  * token store, write_index.fill_, static_pos += 1).  Any of rows/write_index/
  * pos/step may be null to skip that update (rows needs step). */

@@ -1013,7 +1013,7 @@ __global__ __launch_bounds__(256) void argmax_step_kernel(FinArgs a) {
     const int64_t tok = (int64_t)(0xFFFFFFFFu - (unsigned)(part[tid][0] & 0xFFFFFFFFu));
     a.token[tid] = tok;
     if (a.rows != nullptr && s >= 0 && s < a.n_rows) a.rows[tid * a.rows_sb + s] = tok;
-    if (a.pos != nullptr) a.pos[tid] = p + 1;
+    if (a.pos != nullptr && p >= 0) a.pos[tid] = p + 1;  // a parked row stays parked
   }
   if (tid == 0) {
     if (a.write_index != nullptr) a.write_index[0] = wi + 1;

@@ -517,7 +517,7 @@ __global__ __launch_bounds__(1024) void wide_argmax_step_kernel(WideFinArgs a) {
       const int64_t tok = (int64_t)(0xFFFFFFFFu - (unsigned)(k & 0xFFFFFFFFu));
       a.token[b] = tok;
       if (a.rows != nullptr && s >= 0 && s < a.n_rows) a.rows[b * a.rows_sb + s] = tok;
-      if (a.pos != nullptr) a.pos[b] += 1;
+      if (a.pos != nullptr && a.pos[b] >= 0) a.pos[b] += 1;  // a parked row stays parked
     }
   }
   if (threadIdx.x == 0) {

@@ -180,7 +180,7 @@ class PagedDecodeEngine(DecodeEngine):
         ctx["logits"].copy_(logits)
         ctx["token"].copy_(nxt)
         ctx["rows"].index_copy_(1, ctx["step"], nxt.unsqueeze(1))
-        pos.add_(1)
+        pos.add_(pos >= 0)  # a parked row stays parked
         ctx["step"].add_(1)
 
     def capture_paged(self, ctx):

@@ -282,7 +282,8 @@ def argmax_step(keys: torch.Tensor, token: torch.Tensor, rows: torch.Tensor | No
                 step: torch.Tensor | None = None, write_index: torch.Tensor | None = None,
                 pos: torch.Tensor | None = None) -> None:
     """token <- argmax from the lm_head keys; rows[:, step] <- token; step,
-    write_index and pos advance by one (each optional)."""
+    write_index and pos advance by one (each optional; a negative pos, a
+    parked row's, stays)."""
     _check("keys", keys, torch.int64)
     b, n_blocks = keys.shape
     _batch(b)

@@ -158,7 +158,7 @@ def rms_lm_head(x: torch.Tensor, norm_w: torch.Tensor, eps: float, w_lm: Tiles,
 def argmax_step(keys: torch.Tensor, token: torch.Tensor, rows: torch.Tensor, step: torch.Tensor,
                 write_index: torch.Tensor | None, pos: torch.Tensor) -> None:
     """token <- argmax from the lm_head keys; rows[:, step] <- token; step,
-    write_index (if any) and pos advance by one."""
+    write_index (if any) and pos advance by one (a parked row's stays)."""
     b, n_blocks = keys.shape
     _batch(b)
     for name, t in (("keys", keys), ("token", token), ("rows", rows), ("step", step), ("pos", pos)):

@@ -154,3 +154,22 @@ def test_continuous_batching_at_sixteen_rows(dev):
     for i in (0, 3, 9, 16):
         alone = eng.serve([prompts[i], prompts[0]], [news[i], news[0]], max_batch=16)[0]
         assert torch.equal(got[i].cpu(), alone.cpu()), f"request {i}"
+
+
+@pytest.mark.parametrize("batch", [1, 3, 5, 33])
+def test_parked_rows_stay_parked(dev, batch):
+    """Every step body (fused, wide, torch projections): a row at slot -1 is
+    still there after replays, the others advance."""
+    cfg = Qwen2Config(layers=1, vocab=4096)
+    eng = PagedDecodeEngine(cfg, init_weights(cfg, dev, seed=2), dev)
+    kv = eng.new_paged_cache(batch, batch, 64, 1)
+    for r in range(1, batch):
+        kv.map_row(r, 64)
+    ctx = eng.make_paged_context(kv, batch, 4)
+    eng.capture_paged(ctx)
+    ctx["pos"].copy_(torch.arange(batch, device=dev) - 1)
+    print(f"[paged parked] B={batch}", flush=True)
+    for _ in range(3):
+        ctx["graph"].replay()
+    assert ctx["pos"].tolist() == [-1] + [r + 2 for r in range(1, batch)]
+    assert int(ctx["step"]) == 3
