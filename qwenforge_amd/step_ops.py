@@ -60,18 +60,25 @@ class Tiles:
         return (self.n, self.k)
 
 
-def pack_weight(w: torch.Tensor, layout: int = PACK_PLAIN) -> Tiles:
+def pack_weight(w: torch.Tensor, layout: int = PACK_PLAIN, into: Tiles | None = None) -> Tiles:
     """Repack a (N, K) fp16 weight (torch Linear layout) into MFMA tiles on its
-    device (one launch; a load-time step with no counterpart in the reference)."""
+    device (one launch; a load-time step with no counterpart in the reference).
+    The tiles are a copy: after a change of ``w``, ``into`` = its tiles packs
+    them anew in place, so that captured graphs follow."""
     _check("w", w)
     if w.dim() != 2 or w.stride(1) != 1:
         raise ValueError("w must be 2-D with unit inner stride")
     n, k = w.shape
-    out = torch.empty(n * k, device=w.device, dtype=torch.float16)
+    if into is None:
+        out = torch.empty(n * k, device=w.device, dtype=torch.float16)
+    elif (into.n, into.k, into.layout) != (n, k, layout) or into.data.device != w.device:
+        raise ValueError(f"into must hold ({n}, {k}) tiles with row map {layout} on {w.device}")
+    else:
+        out = into.data
     rc = _lib.load().qf_pack_weight(w.data_ptr(), w.stride(0), out.data_ptr(), n, k, layout,
                                     _stream(w.device))
     _lib.check(rc, "qf_pack_weight")
-    return Tiles(out, n, k, layout)
+    return Tiles(out, n, k, layout) if into is None else into
 
 
 def _check(name: str, t: torch.Tensor, dtype=torch.float16) -> None:

@@ -181,3 +181,51 @@ def test_wide_step_matches_torch_step(dev, batch, paged):
     print(f"[wide vs torch step B={batch}] max|dlogit| {(lw - lt).abs().max():.3e}", flush=True)
     assert (lw - lt).abs().max().item() <= LOGIT_TOL
     assert torch.equal(pw, pt) and sw == st and (cw - ct).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("batch", [3, 5, 16])
+def test_decode_follows_weights_changed_in_place(dev, batch):
+    """Other weights copied over an engine's: generate gives a fresh engine's
+    tokens on a reused graph (dense) and a new one (paged), as the torch
+    projections did at 5..32 rows; 3 rows, and a context of the caller's own
+    between replays, after ``repack_weights``."""
+    cfg = Qwen2Config(layers=2, vocab=4096)
+    gen = torch.Generator().manual_seed(batch)
+    ids = torch.randint(0, cfg.vocab, (batch, 20), generator=gen).to(dev)
+    other = init_weights(cfg, dev, seed=22)
+
+    def overwrite(w, source):
+        for to, frm in zip([w] + w["layers"], [source] + source["layers"]):
+            for name, t in to.items():
+                if isinstance(t, torch.Tensor):
+                    t.data.copy_(frm[name])
+
+    print(f"[repack] B={batch}", flush=True)
+    for paged in (False, True):
+        def run(engine):
+            return engine.generate_paged(list(ids), 12) if paged else engine.generate(ids, 12)
+
+        kind = PagedDecodeEngine if paged else DecodeEngine
+        eng = kind(cfg, init_weights(cfg, dev, seed=21), dev)
+        first, want = run(eng), run(kind(cfg, other, dev))
+        assert not torch.equal(first, want)
+        overwrite(eng.w, other)
+        if batch < wide_ops.MIN_BATCH:
+            eng.repack_weights()
+        assert torch.equal(run(eng), want)
+        assert paged or eng.captures == 1
+    ctx = eng._ctx
+    logits = []
+    for change in (False, True):
+        if change:  # the layers alone: the embedding is read where it lies
+            back = init_weights(cfg, dev, seed=21)
+            for to, frm in zip(eng.w["layers"], back["layers"]):
+                for name in ("qkv_weight", "o_weight", "gate_up_weight", "down_weight"):
+                    to[name].copy_(frm[name])
+            eng.repack_weights()
+        ctx["pos"].fill_(20)
+        ctx["step"].fill_(1)
+        ctx["token"].fill_(7)
+        ctx["graph"].replay()
+        logits.append(ctx["logits"].clone())
+    assert not torch.equal(*logits)
