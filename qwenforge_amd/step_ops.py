@@ -75,8 +75,9 @@ def pack_weight(w: torch.Tensor, layout: int = PACK_PLAIN, into: Tiles | None = 
         raise ValueError(f"into must hold ({n}, {k}) tiles with row map {layout} on {w.device}")
     else:
         out = into.data
-    rc = _lib.load().qf_pack_weight(w.data_ptr(), w.stride(0), out.data_ptr(), n, k, layout,
-                                    _stream(w.device))
+    with torch.cuda.device(w.device):
+        rc = _lib.load().qf_pack_weight(w.data_ptr(), w.stride(0), out.data_ptr(), n, k, layout,
+                                        _stream(w.device))
     _lib.check(rc, "qf_pack_weight")
     return Tiles(out, n, k, layout) if into is None else into
 

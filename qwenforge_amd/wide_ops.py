@@ -5,7 +5,8 @@ The step of ``step_ops`` (SE:896-982) for wider batches: every weight is
 ``step_ops.Tiles``, o_proj takes the attention's merged output
 (``ops.flash_decode_attention``), and the long down projection is split over
 workgroups through the caller's ``make_wide_scratch``.  Like there, every
-function launches on the current HIP stream; nothing computes on the host.
+function launches on the current HIP stream (of its operands' device, whichever
+is current); nothing computes on the host.
 """
 
 from __future__ import annotations
@@ -62,10 +63,11 @@ def _rms_qkv(x, norm_w, eps, w_qkv, bias, positions, caches, slots, q_out, kvh, 
         raise ValueError("pos must be contiguous (B,)")
     if inv.shape != (d // 2,) or not inv.is_contiguous():
         raise ValueError(f"inv_freq must be contiguous ({d // 2},)")
-    rc = _lib.load().qf_wide_qkv(
-        x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr, _ptr(bias), pos.data_ptr(),
-        inv.data_ptr(), *caches, *slots, q_out.data_ptr(), q_out.stride(0), q_out.stride(1),
-        b, hidden, qh, kvh, d, cap, _stream(x.device))
+    with torch.cuda.device(x.device):
+        rc = _lib.load().qf_wide_qkv(
+            x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr, _ptr(bias), pos.data_ptr(),
+            inv.data_ptr(), *caches, *slots, q_out.data_ptr(), q_out.stride(0), q_out.stride(1),
+            b, hidden, qh, kvh, d, cap, _stream(x.device))
     _lib.check(rc, "qf_wide_qkv")
 
 
@@ -115,9 +117,10 @@ def gemv_residual(inp: torch.Tensor, w: Tiles, hidden: torch.Tensor, scratch) ->
     _check("ticket", ticket, torch.int32)
     if part.numel() < n // 16 * lib.qf_wide_splits(k) * -(-b // 16) * 256 or ticket.numel() < n // 16:
         raise ValueError("scratch too small for this weight and batch (make_wide_scratch)")
-    rc = lib.qf_wide_gemv_residual(inp.data_ptr(), in_sb, w_ptr, hidden.data_ptr(), h_sb,
-                                   part.data_ptr(), ticket.data_ptr(), b, k, n,
-                                   _stream(inp.device))
+    with torch.cuda.device(inp.device):
+        rc = lib.qf_wide_gemv_residual(inp.data_ptr(), in_sb, w_ptr, hidden.data_ptr(), h_sb,
+                                       part.data_ptr(), ticket.data_ptr(), b, k, n,
+                                       _stream(inp.device))
     _lib.check(rc, "qf_wide_gemv_residual")
 
 
@@ -131,8 +134,9 @@ def rms_gate_up_swiglu(x: torch.Tensor, norm_w: torch.Tensor, eps: float, w_gate
     _check("norm_w", norm_w)
     w_ptr = _tiles("w_gate_up", w_gate_up, 2 * inter, hidden, PACK_SWIGLU)
     ho_sb = _rows("h_out", h_out, b, inter)
-    rc = _lib.load().qf_wide_gate_up(x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr,
-                                     h_out.data_ptr(), ho_sb, b, hidden, inter, _stream(x.device))
+    with torch.cuda.device(x.device):
+        rc = _lib.load().qf_wide_gate_up(x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr,
+                                         h_out.data_ptr(), ho_sb, b, hidden, inter, _stream(x.device))
     _lib.check(rc, "qf_wide_gate_up")
 
 
@@ -149,9 +153,10 @@ def rms_lm_head(x: torch.Tensor, norm_w: torch.Tensor, eps: float, w_lm: Tiles,
     _check("keys", keys, torch.int64)
     if keys.dim() != 2 or keys.shape[0] != b or not keys.is_contiguous():
         raise ValueError("keys must be contiguous (B, n_blocks) int64")
-    rc = _lib.load().qf_wide_lm_head(x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr,
-                                     logits.data_ptr(), lg_sb, keys.data_ptr(), keys.shape[1], b,
-                                     hidden, vocab, _stream(x.device))
+    with torch.cuda.device(x.device):
+        rc = _lib.load().qf_wide_lm_head(x.data_ptr(), x_sb, norm_w.data_ptr(), float(eps), w_ptr,
+                                         logits.data_ptr(), lg_sb, keys.data_ptr(), keys.shape[1], b,
+                                         hidden, vocab, _stream(x.device))
     _lib.check(rc, "qf_wide_lm_head")
 
 
@@ -169,8 +174,9 @@ def argmax_step(keys: torch.Tensor, token: torch.Tensor, rows: torch.Tensor, ste
         raise ValueError("rows must be (B, T) with unit inner stride, keys contiguous")
     if write_index is not None:
         _check("write_index", write_index, torch.int64)
-    rc = _lib.load().qf_wide_argmax_step(keys.data_ptr(), n_blocks, b, token.data_ptr(),
-                                         rows.data_ptr(), rows.stride(0), rows.shape[1],
-                                         step.data_ptr(), _ptr(write_index), pos.data_ptr(),
-                                         _stream(keys.device))
+    with torch.cuda.device(keys.device):
+        rc = _lib.load().qf_wide_argmax_step(keys.data_ptr(), n_blocks, b, token.data_ptr(),
+                                             rows.data_ptr(), rows.stride(0), rows.shape[1],
+                                             step.data_ptr(), _ptr(write_index), pos.data_ptr(),
+                                             _stream(keys.device))
     _lib.check(rc, "qf_wide_argmax_step")

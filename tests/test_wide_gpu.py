@@ -7,12 +7,14 @@ outputs match bit for bit; random ones agree to a few fp16 ulps (the bound of
 the 1..4-row kernels' tests).
 """
 
+import types
+
 import pytest
 import torch
 
 import oracle.step as ost
 from oracle.rope import inv_freq, rope_cos_sin
-from qwenforge_amd import step_ops, wide_ops
+from qwenforge_amd import _lib, step_ops, wide_ops
 from qwenforge_amd.engine import DecodeEngine
 from qwenforge_amd.model import Qwen2Config, init_weights
 from qwenforge_amd.paged_engine import PagedDecodeEngine
@@ -229,3 +231,46 @@ def test_decode_follows_weights_changed_in_place(dev, batch):
         ctx["graph"].replay()
         logits.append(ctx["logits"].clone())
     assert not torch.equal(*logits)
+
+
+def test_every_launch_runs_with_its_operands_device_current(dev, monkeypatch):
+    """An engine on another device than the current one: each call of the wide
+    step and of the packing enters its operands' device first (the null stream
+    a launch names is the current device's)."""
+    inside, calls = [], []
+
+    class Guard(torch.cuda.device):
+        def __enter__(self):
+            inside.append(self.idx)
+            return super().__enter__()
+
+        def __exit__(self, *exc):
+            inside.pop()
+            return super().__exit__(*exc)
+
+    class Lib(types.SimpleNamespace):
+        def __getattr__(self, name):
+            def call(*args):
+                if name != "qf_wide_splits":
+                    calls.append((name, list(inside)))
+                return int(name == "qf_wide_splits")
+            return call
+
+    f16 = dict(device=dev, dtype=torch.float16)
+    x, nw, q = torch.zeros(5, 64, **f16), torch.zeros(64, **f16), torch.zeros(5, 1, 64, **f16)
+    pos, inv = torch.zeros(5, device=dev).long(), torch.zeros(32, device=dev)
+    cache, pool = torch.zeros(5, 1, 8, 64, **f16), torch.zeros(5, 1, 64, 64, **f16)
+    table = torch.zeros(5, 1, device=dev, dtype=torch.int32)
+    keys, rows = torch.zeros(5, 2, device=dev).long(), torch.zeros(5, 2, device=dev).long()
+    scratch = wide_ops.make_wide_scratch(5, 64, 64, dev)
+    monkeypatch.setattr(_lib, "load", Lib)
+    monkeypatch.setattr(torch.cuda, "device", Guard)
+    w_qkv, w, w_gu = (step_ops.pack_weight(torch.zeros(n, 64, **f16), layout) for n, layout in (
+        (192, step_ops.PACK_ROPE), (64, step_ops.PACK_PLAIN), (128, step_ops.PACK_SWIGLU)))
+    wide_ops.rms_qkv_rope_append(x, nw, EPS, w_qkv, None, (pos, inv), cache, cache, pos[:1], q)
+    wide_ops.rms_qkv_rope_append_paged(x, nw, EPS, w_qkv, None, (pos, inv), pool, pool, table, pos, q)
+    wide_ops.gemv_residual(x, w, x, scratch)
+    wide_ops.rms_gate_up_swiglu(x, nw, EPS, w_gu, x)
+    wide_ops.rms_lm_head(x, nw, EPS, w, x, keys)
+    wide_ops.argmax_step(keys, pos, rows, pos[:1], None, pos)
+    assert len(calls) == 9 and all(where == [x.device.index] for _, where in calls), calls
