@@ -35,6 +35,7 @@ namespace qf {
 namespace step {
 
 constexpr int kPad = 8;            // halves of padding per staged row
+constexpr int kNt = 2;             // non-temporal bit of a buffer access
 constexpr int kNormBlk = kMaxNormK / 32 / kNW;  // k blocks per wave of a normalised row (max)
 
 // Columns of 16 for kRows staged rows per wave (4 * kRows rows in all).
@@ -97,8 +98,27 @@ __device__ __forceinline__ f16x8 wide_operand(const f16* xs, int K, int kb, int 
   return *reinterpret_cast<const f16x8*>(xs + row * (K + kPad) + 32 * kb + 8 * (lane >> 4));
 }
 
+// The weight tiles of k blocks [kb0, kb0 + n) of row block rb, zeros past n: a
+// real tile re-read there could hold infinities, which zero columns turn into
+// NaN.  A surplus block is a (non-temporal) buffer load past its range, so it
+// costs neither traffic nor selects on its registers (MI355X, a step of 12 rows
+// and 24 layers: 751.6 us against 753.9 with selects, 749.9 with re-read tiles;
+// the attention half at 4 rows 319 against 323 and 322).  rb is wave-uniform; one past nrb reads zeros.
+template <int kBlk>
+__device__ __forceinline__ void share_tiles(f16x8 (&wa)[kBlk], const f16* w, int nkb, int nrb,
+                                            int rb, int kb0, int n, int lane) {
+  const __amdgpu_buffer_rsrc_t r =
+      buffer_rsrc(w + (int64_t)rb * nkb * 512, rb < nrb ? nkb * 1024 : 0);
+#pragma unroll
+  for (int t = 0; t < kBlk; ++t)
+    wa[t] = __builtin_bit_cast(
+        f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                   r, t < n ? ((kb0 + t) * 64 + lane) * 16 : 0x7ffffff0, 0, kNt));
+}
+
 // This wave's k blocks [kb0, kb0 + n) of one row block against every column
-// block; the operands of all blocks are read before the first MFMA.
+// block; the operands of all blocks are read before the first MFMA.  A block
+// past n multiplies zeros on both sides (share_tiles, and here).
 template <int kRows, int kBlk>
 __device__ __forceinline__ void wide_mfma(const f16x8 (&wa)[kBlk], const f16* xs, int K, int kb0,
                                           int n, int lane, f32x4 (&acc)[col_blocks(kRows)]) {
@@ -157,8 +177,7 @@ __global__ __launch_bounds__(kNT) void wide_qkv_kernel(QkvArgs a) {
     }
   }
   f16x8 wa[kNormBlk];
-#pragma unroll
-  for (int t = 0; t < kNormBlk; ++t) wa[t] = tile_load(a.w, nkb, rb, min(kb0 + t, nkb - 1), lane);
+  share_tiles(wa, a.w, nkb, (int)gridDim.x, rb, kb0, n, lane);
   bool in_range = slot >= 0 && slot < a.cap;
   int64_t kro, vro;
   if (kPaged) {
@@ -345,10 +364,7 @@ __global__ __launch_bounds__(kNT) void wide_gate_up_kernel(GateUpArgs a) {
   wide_load<kRows>(st, a.x, a.x_sb, a.B, K / 8, a.norm_w);
   f16x8 wa[kRB][kNormBlk];
 #pragma unroll
-  for (int r = 0; r < kRB; ++r)
-#pragma unroll
-    for (int t = 0; t < kNormBlk; ++t)
-      wa[r][t] = tile_load(a.w, nkb, min(rb0 + r, nrb - 1), min(kb0 + t, nkb - 1), lane);
+  for (int r = 0; r < kRB; ++r) share_tiles(wa[r], a.w, nkb, nrb, rb0 + r, kb0, n, lane);
   wide_finish<kRows>(st, K, a.eps, xs);
 #pragma unroll
   for (int r = 0; r < kRB; ++r) {
@@ -429,7 +445,11 @@ __global__ __launch_bounds__(kNT) void wide_lm_head_kernel(WideLmArgs a) {
   }
   for (int i = 0; i < items; ++i) {
     load_stage(i + 1, nxt);
-    const int ch = i % nch, n = min(KC, nkb - ch * KC);
+    const int ch = i % nch, n = __builtin_amdgcn_readfirstlane(min(KC, nkb - ch * KC));
+    if (n < KC)  // the tiles past a short stage re-read real ones, which may hold infinities
+#pragma unroll
+      for (int t = 1; t < KC; ++t)
+        if (t >= n) cur[t] = zero8();
 #pragma unroll
     for (int t = 0; t < KC; ++t)
 #pragma unroll

@@ -274,3 +274,45 @@ def test_every_launch_runs_with_its_operands_device_current(dev, monkeypatch):
     wide_ops.rms_lm_head(x, nw, EPS, w, x, keys)
     wide_ops.argmax_step(keys, pos, rows, pos[:1], None, pos)
     assert len(calls) == 9 and all(where == [x.device.index] for _, where in calls), calls
+
+
+@pytest.mark.parametrize("hidden", [64, 96, 160, HIDDEN])
+@pytest.mark.parametrize("batch", [3, 5, 20])
+def test_infinite_weights_stay_infinities(dev, batch, hidden):
+    """One infinite weight in every k block in turn (k blocks past a wave's
+    share re-read such a tile): its output row is an infinity of the row's
+    sign, as in torch, and the others are untouched."""
+    x = torch.ones(batch, hidden, dtype=torch.float16)
+    x[1] = -1
+    x, nw = x.to(dev), torch.ones(hidden, **dict(device=dev, dtype=torch.float16))
+    pos, inv = torch.zeros(batch, device=dev).long(), inv_freq(D, 1e6).to(dev)
+    print(f"[wide inf] B={batch} hidden={hidden}", flush=True)
+    want = torch.full((batch,), float("inf"), device=dev, dtype=torch.float16)
+    want[1] = -want[1]
+    for kb in range(hidden // 32):
+        w = torch.zeros(256, hidden, device=dev, dtype=torch.float16)
+        w[128 + 32 * (kb % 2), 32 * kb + 5] = float("inf")  # a V row (kv head 0: rows 128..191)
+        if batch >= wide_ops.MIN_BATCH:
+            logits = torch.zeros(batch, 256, device=dev, dtype=torch.float16)
+            wide_ops.rms_lm_head(x, nw, EPS, step_ops.pack_weight(w), logits,
+                                 torch.zeros(batch, 3, device=dev).long())
+            assert torch.equal(logits[:, 128 + 32 * (kb % 2)], want), kb
+            assert int((logits != 0).sum()) == batch
+        qkv = w[:192].contiguous()
+        kc, vc = (torch.zeros(batch, 1, 4, D, device=dev, dtype=torch.float16) for _ in range(2))
+        q = torch.zeros(batch, 1, D, device=dev, dtype=torch.float16)
+        tiles = step_ops.pack_weight(qkv, step_ops.PACK_ROPE)
+        if batch >= wide_ops.MIN_BATCH:
+            wide_ops.rms_qkv_rope_append(x, nw, EPS, tiles, None, (pos, inv), kc, vc, pos[:1], q)
+        else:
+            step_ops.rms_qkv_rope_append(x, nw, EPS, tiles, None, None, None, kc, vc, pos[:1], q,
+                                         positions=(pos, inv))
+        assert torch.equal(vc[:, 0, 0, 32 * (kb % 2)], want), kb
+        assert int((vc != 0).sum()) == batch and not bool(q.any()) and not bool(kc.any())
+        # Gate rows 1 and 0 infinite against up rows of ones: silu(inf) * 1.
+        gu = torch.zeros(32, hidden, device=dev, dtype=torch.float16)
+        gu[3, 32 * kb + 5], gu[16 + 3] = float("inf"), 1 / hidden
+        h = torch.zeros(batch, 16, device=dev, dtype=torch.float16)
+        packed = step_ops.pack_weight(gu, step_ops.PACK_SWIGLU)
+        (wide_ops if batch >= wide_ops.MIN_BATCH else step_ops).rms_gate_up_swiglu(x, nw, EPS, packed, h)
+        assert bool(torch.isposinf(h[[0, 2], 3]).all()) and not bool(h[:, :3].any()), kb
