@@ -10,6 +10,7 @@ tests, so they are within the sum of the two of each other; the shallow model
 here stays far inside (fp16 roundings of two layers).
 """
 
+import numpy as np
 import pytest
 import torch
 
@@ -141,3 +142,37 @@ def test_layouts_it_does_not_take(dev, weights):
     layers[1]["o_weight"] = weights["layers"][1]["o_weight"].float()
     assert prefill_ops.layer_table(CFG, layers, caches, dev, shape) is None
     assert prefill_ops.workspace_bytes(Qwen2Config(hidden=960, heads=15, kv_heads=3), 8) < 0
+
+
+def test_swiglu_rounds_every_gate_correctly(dev):
+    """A layer whose h is silu(v) of chosen fp16 values: token t holds one
+    number, 2^10 at place t, which the norm turns into 32 exactly; gate weights
+    v / 32 and up weights 1 / 32 in that column, the down projection picks h
+    out.  Every fp16 v from 2^-8 to the largest, both signs, against silu in
+    fp64 rounded once (which F.silu gives for all of them)."""
+    cfg = Qwen2Config(hidden=1024, heads=16, kv_heads=2, intermediate=1024, layers=1, vocab=64)
+    tokens, n = 64, 1024
+    bits = torch.arange(0x1C00, 0x7C00, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    v = torch.cat([bits, -bits])
+    v = torch.cat([v, v[:tokens * (n - tokens) - v.numel()]]).view(tokens, n - tokens).to(dev)
+    gate_up = torch.zeros(2 * n, n, device=dev, dtype=torch.float16)
+    gate_up[tokens:n, :tokens] = (v / 32).t()
+    assert torch.equal(gate_up[tokens:n, :tokens].t() * 32, v)
+    gate_up[n:, :tokens] = 1 / 32
+    zeros = lambda *s: torch.zeros(*s, device=dev, dtype=torch.float16)  # noqa: E731
+    layer = {"input_norm": zeros(n) + 1, "post_norm": zeros(n) + 1, "qkv_bias": None,
+             "qkv_weight": zeros(cfg.qkv_width, n), "o_weight": zeros(n, n),
+             "gate_up_weight": gate_up, "down_weight": torch.eye(n, device=dev).half()}
+    caches = [(zeros(1, 2, 64, 64), zeros(1, 2, 64, 64))]
+    hidden = zeros(tokens, n)
+    hidden[:, :tokens].fill_diagonal_(1024.0)
+    table = prefill_ops.layer_table(cfg, [layer], caches, dev, (1, 2, tokens, 64))
+    inv = torch.zeros(32, device=dev)
+    prefill_ops.prefill_layers(cfg, table, hidden, 1, tokens, inv)
+    # numpy rounds fp64 to fp16 once (torch by way of fp32).
+    exact = v.double().cpu().numpy()
+    want = torch.from_numpy((exact / (1 + np.exp(-exact))).astype(np.float16)).to(dev)
+    got = hidden[:, tokens:]
+    print(f"[prefill silu] {int((got != want).sum())} of {want.numel()} differ", flush=True)
+    assert torch.equal(torch.nn.functional.silu(v), want)
+    assert torch.equal(got, want)
