@@ -34,7 +34,9 @@ int qf_wide_qkv(const void* x, int64_t x_sb, const void* norm_w, float eps, cons
                 int64_t slot_sb, void* q_out, int64_t qo_sb, int64_t qo_sh, int B, int hidden,
                 int QH, int KVH, int D, int cap, void* stream);
 
-/* Workgroups that share one row block's k range in qf_wide_gemv_residual. */
+/* Workgroups that share one row block's k range in qf_wide_gemv_residual;
+ * QF_ERR_UNSUPPORTED for a K that it does not take (a multiple of 32, up to
+ * 3.3 million). */
 int qf_wide_splits(int K);
 
 /* hidden <- fp16(hidden + fp16(inp @ w^T)), in place (o_proj SE:973-974,

@@ -644,7 +644,10 @@ constexpr int kGemvBlk = 8, kSplitBlk = 5;
 extern "C" int qf_wide_splits(int K) {
   if (K < 32 || K % 32) return QF_ERR_UNSUPPORTED;
   const int nkb = K / 32, per = nkb <= kNW * kGemvBlk ? kGemvBlk : kSplitBlk;
-  return (nkb + kNW * per - 1) / (kNW * per);
+  const int splits = (nkb - 1) / (kNW * per) + 1;
+  // The kernel cuts its shares at (share * nkb) / shares in 32 bits.
+  if ((int64_t)kNW * splits * nkb > 0x7fffffff) return QF_ERR_UNSUPPORTED;
+  return splits;
 }
 
 template <int kBlk, bool kSplit>
@@ -661,7 +664,7 @@ extern "C" int qf_wide_gemv_residual(const void* inp, int64_t in_sb, const void*
   if (!inp || !w || !hidden) return QF_ERR_INVALID_ARG;
   if (!al16(inp) || !al16(w) || (in_sb & 7) || !al8(hidden) || (h_sb & 3)) return QF_ERR_INVALID_ARG;
   const int splits = qf_wide_splits(K);
-  if (splits > 65535) return QF_ERR_UNSUPPORTED;
+  if (splits < 0) return splits;
   if (splits > 1 && (!part || !ticket || !al16(part))) return QF_ERR_INVALID_ARG;
   WideGemvArgs a;
   a.inp = static_cast<const f16*>(inp); a.in_sb = in_sb;

@@ -279,3 +279,25 @@ def test_pack_weight_rejects_bad_arguments():
     assert lib.qf_pack_weight(None, 896, 16, 1152, 896, 0, None) == -1
     assert lib.qf_pack_weight(16, 800, 16, 1152, 896, 0, None) == -1     # row stride < K
     assert lib.qf_pack_weight(18, 896, 16, 1152, 896, 0, None) == -1     # misaligned
+
+
+@pytest.mark.parametrize("k", [32, 96, 1024, 1056, 4864, 8192, 1 << 20, 3_300_000, 3_315_840])
+def test_wide_gemv_shares_cover_k(k):
+    """The shares of a long k as the kernel cuts them, in 32-bit arithmetic: in
+    order, whole, and within the blocks a wave loads."""
+    np = pytest.importorskip("numpy")
+    splits, nkb = _lib.load().qf_wide_splits(k), k // 32
+    assert splits >= 1
+    cuts = [np.int32(0)]
+    with np.errstate(over="raise"):
+        for mine in range(4 * splits):
+            cuts.append(np.int32(mine + 1) * np.int32(nkb) // np.int32(4 * splits))
+    assert cuts[-1] == nkb
+    assert 0 <= min(np.diff(cuts)) and max(np.diff(cuts)) <= (8 if splits == 1 else 5)
+
+
+def test_wide_gemv_rejects_a_k_past_its_arithmetic():
+    lib = _lib.load()
+    for k in (0, 48, 3_315_872, 40_000_000, 0x7FFFFFE0):
+        assert lib.qf_wide_splits(k) == -2, k
+        assert lib.qf_wide_gemv_residual(16, 64, 16, 16, 16, 16, 16, 5, k, 16, None) == -2, k
