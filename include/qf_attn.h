@@ -137,6 +137,11 @@ int qf_decode_attn_shared(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_s
  */
 int qf_decode_waves(int B, int KVH, int G, int cap, int splits, int fused);
 
+/* The same for qf_decode_attn_shared with a ticket, a kv_last per row and no
+ * bias: 1 if it shares its workgroups out by the rows' lengths (merge mode 4),
+ * 0 if it is qf_decode_attn's launch. */
+int qf_decode_shares(int B, int KVH, int G, int cap, int splits);
+
 /*
  * qf_decode_attn without caller scratch.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under hipGraph

@@ -956,6 +956,21 @@ extern "C" int qf_decode_waves(int B, int KVH, int G, int cap, int splits, int f
   return pick_waves(a, merge_mode(splits, fused != 0));
 }
 
+extern "C" int qf_decode_shares(int B, int KVH, int G, int cap, int splits) {
+  if (G < 1 || G > kMaxG || B < 1 || KVH < 1 || cap < 1 || splits < 1 || splits > 65535)
+    return QF_ERR_INVALID_ARG;
+  DecodeArgs a{};
+  a.B = B;
+  a.KVH = KVH;
+  a.G = G;
+  a.cap = cap;
+  a.splits = splits;
+  int64_t last = 0;
+  a.kv_last = &last;  // only whether there is one
+  a.kv_last_sb = 1;
+  return merge_mode(splits, true) == kFused && shares_by_length(a) ? 1 : 0;
+}
+
 extern "C" int qf_decode_split(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sg,
                                const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                                const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,

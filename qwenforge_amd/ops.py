@@ -208,14 +208,20 @@ def ticket_size(batch: int, kv_heads: int, splits: int) -> int:
 
 
 def decode_kernel_name(batch: int, kv_heads: int, groups: int, capacity: int, splits: int,
-                       fused: bool, bias: str = "vec", paged: bool = False) -> str:
+                       fused: bool, bias: str = "vec", paged: bool = False,
+                       row_bounds: bool = False) -> str:
     """Name of the split-kernel instance a decode call launches, from the
-    library's own launch plan (``qf_decode_waves``): decode_split_kernel<waves,
-    bias (0 none, 1 16-byte vector, 2 scalar), mode (0 direct, 1 partial, 2
-    single-launch merge), paged>."""
-    waves = _lib.load().qf_decode_waves(batch, kv_heads, groups, capacity, splits, int(fused))
+    library's own launch plan (``qf_decode_waves``, ``qf_decode_shares``):
+    decode_split_kernel<waves, bias (0 none, 1 16-byte vector, 2 scalar), mode
+    (0 direct, 1 partial, 2 single-launch merge, 4 with the workgroups shared
+    out by the rows' lengths), paged>.  ``row_bounds``: the call has a
+    ``kv_last`` per row and may share (``share_rows``)."""
+    lib = _lib.load()
+    waves = lib.qf_decode_waves(batch, kv_heads, groups, capacity, splits, int(fused))
     _lib.check(min(waves, 0), "qf_decode_waves")
     mode = 0 if splits == 1 else (2 if fused else 1)
+    if mode == 2 and row_bounds and bias == "none":
+        mode = 4 if lib.qf_decode_shares(batch, kv_heads, groups, capacity, splits) else 2
     kind = {"none": 0, "vec": 1, "scalar": 2}[bias]
     return f"qf::decode_split_kernel<{waves}, {kind}, {mode}, {str(paged).lower()}>"
 

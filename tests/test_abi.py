@@ -301,3 +301,38 @@ def test_wide_gemv_rejects_a_k_past_its_arithmetic():
     for k in (0, 48, 3_315_872, 40_000_000, 0x7FFFFFE0):
         assert lib.qf_wide_splits(k) == -2, k
         assert lib.qf_wide_gemv_residual(16, 64, 16, 16, 16, 16, 16, 5, k, 16, None) == -2, k
+
+
+@pytest.mark.parametrize("b,cap,splits,fused,bias,bounds,mode", [
+    (16, 6016, 8, True, "none", True, 4),    # ragged paged serving
+    (16, 1536, 8, True, "none", True, 4),    # six tiles of capacity a split
+    (16, 1535, 8, True, "none", True, 2),
+    (16, 6016, 9, True, "none", True, 2),    # nine splits
+    (64, 6016, 2, True, "none", True, 4),
+    (65, 6016, 2, True, "none", True, 2),    # 65 rows
+    (1, 6016, 8, True, "none", True, 2),     # one row
+    (16, 6016, 8, True, "none", False, 2),   # one bound for all, or even splits asked for
+    (16, 6016, 8, True, "vec", True, 2),     # a bias
+    (16, 6016, 8, False, "none", True, 1),   # two launches
+    (16, 6016, 1, True, "none", True, 0),
+])
+def test_decode_kernel_name_follows_the_shared_form(b, cap, splits, fused, bias, bounds, mode):
+    from qwenforge_amd import ops
+
+    name = ops.decode_kernel_name(b, 2, 7, cap, splits, fused, bias, paged=True, row_bounds=bounds)
+    assert name.split(", ")[2] == str(mode), name
+
+
+def test_shared_decode_rejects_what_the_even_one_rejects():
+    lib = _lib.load()
+    assert lib.qf_decode_shares(4, 2, 0, 64, 1) == -1
+    for shared in ("", "_shared"):
+        def call(q=16, D=64, splits=1):
+            return getattr(lib, "qf_decode_attn" + shared)(
+                q, 0, 0, 0, 16, 0, 0, 0, 16, 0, 0, 0, None, 0, None, 0, 16, 16, 16, splits, None,
+                16, 0, 0, 0, 1, 2, 7, D, 8, 0.125, None)
+
+        assert call(D=128) == -2 and call(q=None) == -1 and call(splits=0) == -1
+        assert getattr(lib, "qf_decode_attn_paged" + shared)(
+            16, 0, 0, 0, 16, 8192, 4096, 64, 16, 8192, 4096, 64, None, 4, 4, 8, 64, None, 0, None, 0,
+            16, 16, 16, 1, None, 16, 0, 0, 0, 1, 2, 7, 64, 0.125, None) == -1
