@@ -72,12 +72,13 @@ def test_paged_prefill_and_decode_match_oracle(dev, page):
     assert ctx["pos"].cpu().tolist() == [n + steps for n in lengths]
 
 
-@pytest.mark.parametrize("max_batch", [2, 5])
-def test_continuous_batching_matches_isolated_requests(dev, max_batch):
-    """Five requests through 2 rows (fused step) or 5 rows (torch-projection
-    step): rows are recycled as requests finish, pages return to the pool."""
+@pytest.mark.parametrize("max_batch,tiles", [(2, True), (5, True), (5, False)])
+def test_continuous_batching_matches_isolated_requests(dev, max_batch, tiles):
+    """Five requests through 2 rows (fused step) or 5 rows (wide step; without
+    tile weights the torch-projection step): rows are recycled as requests
+    finish, pages return to the pool."""
     cfg = Qwen2Config(layers=2)
-    eng = PagedDecodeEngine(cfg, init_weights(cfg, dev, seed=7), dev)
+    eng = PagedDecodeEngine(cfg, init_weights(cfg, dev, seed=7), dev, tile_weights=tiles)
     gen = torch.Generator().manual_seed(3)
     lengths = [40, 100, 7, 64, 130]
     news = [6, 3, 8, 1, 5]
