@@ -45,8 +45,9 @@ int64_t qf_prefill_layers_workspace(int T, int hidden, int QH, int KVH, int D, i
  * the residual stream after the last layer out; each token's rotated K and raw
  * V go to its cache slot.  cu null: B rows of S tokens each.  Otherwise packed
  * rows, cu (B + 1) int32 on the device as in qf_prefill_varlen with S the
- * longest row.  Token i of row b goes to slot i of row b (which the caller
- * sized); with block_table through it, a page outside the pool writing
+ * longest row (a token past it in its row is not appended).  Token i of row b
+ * goes to slot i of row b: every cache holds S slots at least, which the caller
+ * checks; with block_table through it, a page outside the pool writing
  * nothing.  ws: 16-byte aligned, free again when the call's work is done. */
 int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, void* hidden, int T, int B, int S,
                       const int32_t* cu, const float* inv_freq, const int32_t* block_table,

@@ -446,7 +446,8 @@ __global__ __launch_bounds__(256) void prefill_rms_kernel(f16* x, const f16* __r
 
 // Per token of the packed rows: the fp16 RoPE table of its position (the same
 // values as the torch table, student_engine.py:910-915) and where it is
-// appended.  cu == nullptr: rows of S tokens.  One wave per two tokens.
+// appended.  cu == nullptr: rows of S tokens; else rows of at most S, a token
+// past them appending nothing.  One wave per two tokens.
 __global__ __launch_bounds__(256) void prefill_tokens_kernel(const int* cu, int B, int S, int T,
                                                              const float* inv_freq,
                                                              const int32_t* table, int64_t t_sb,
@@ -472,10 +473,10 @@ __global__ __launch_bounds__(256) void prefill_tokens_kernel(const int* cu, int 
   cs[64 * t + i] = (f16)cosf(ang);
   cs[64 * t + 32 + i] = (f16)sinf(ang);
   if (i == 0) {
-    int2 at = make_int2(b, pos);
+    int2 at = make_int2(pos < S ? b : -1, pos);
     if (table != nullptr) {
       const int lp = pos >> log2p;
-      const int page = lp < ppr ? table[b * t_sb + lp] : -1;
+      const int page = pos < S && lp < ppr ? table[b * t_sb + lp] : -1;
       at = make_int2(page >= 0 && page < n_pages ? page : -1, pos & ((1 << log2p) - 1));
     }
     info[t] = at;

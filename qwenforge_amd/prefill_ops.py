@@ -29,7 +29,8 @@ def layer_table(cfg, layers, caches, device, shape):
     """The ``Layer`` array of a model's weights and (K, V) caches, or None if
     any of them has another type, device, layout or size.  ``shape`` is the
     caches' (rows or pages, kv heads, least slots, 64).  Built for each call:
-    no pointer outlives it."""
+    no pointer outlives it.  ``rows`` and ``slots`` of the result are what every
+    cache holds."""
     h, width = cfg.hidden, cfg.qkv_width
     want = (("input_norm", (h,)), ("qkv_weight", (width, h)), ("qkv_bias", (width,)),
             ("o_weight", (h, cfg.heads * cfg.head_dim)), ("post_norm", (h,)),
@@ -38,6 +39,7 @@ def layer_table(cfg, layers, caches, device, shape):
         return None
     table = (Layer * len(layers))()
     rows, heads, slots, dim = shape
+    table.rows, table.slots = rows, min((t.shape[2] for pair in caches for t in pair), default=0)
     for entry, layer, pair in zip(table, layers, caches):
         ptrs = []
         for name, size in want:
@@ -80,6 +82,14 @@ def prefill_layers(cfg, table, hidden: torch.Tensor, rows: int, longest: int,
     ``rows`` rows of ``longest`` tokens, or packed rows of at most that many
     with their offsets ``cu`` (rows + 1) int32 on the device."""
     tokens = hidden.numel() // cfg.hidden
+    if block_table is None and (table.rows != rows or longest > table.slots):
+        raise ValueError(f"caches of {table.rows} rows and {table.slots} slots do not hold "
+                         f"{rows} rows of {longest} tokens")
+    if block_table is not None and (
+            (n_pages, page_size) != (table.rows, table.slots) or block_table.dim() != 2
+            or longest > block_table.shape[1] * page_size):
+        raise ValueError("n_pages and page_size must be the pools' and the table's rows hold "
+                         f"{longest} slots")
     if hidden.dtype != torch.float16 or hidden.device.type != "cuda" or not hidden.is_contiguous():
         raise ValueError("hidden must be a contiguous fp16 device tensor")
     if cu is not None and (cu.dtype != torch.int32 or cu.shape != (rows + 1,)

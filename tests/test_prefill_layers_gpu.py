@@ -259,3 +259,29 @@ def test_layer_exact_on_integers(dev, hidden, heads, kv, inter, tokens):
     assert torch.equal(vc.view(tokens, -1), v)
     att = v.view(tokens, kv, 1, 64).expand(-1, -1, cfg.groups, -1).reshape(tokens, hidden)
     assert torch.equal(got, (x + (att.float() @ w_o.T).half().float()).half())
+
+
+def test_appends_stay_within_the_rows(dev, weights):
+    """A cache that holds fewer rows, slots or pages than the call fills is
+    refused before any launch; a packed row longer than the longest announced
+    appends no further than that (slots past it exist here)."""
+    eng = DecodeEngine(CFG, weights, dev)
+    caches, pools = eng.new_caches(2, 40), [(torch.zeros(4, 2, 64, 64, device=dev).half(),) * 2] * 2
+    hidden = weights["embed"][:40].clone()
+    table = prefill_ops.layer_table(CFG, weights["layers"], caches, dev, (2, 2, 1, 64))
+    paged = prefill_ops.layer_table(CFG, weights["layers"], pools, dev, (4, 2, 64, 64))
+    block_table = torch.zeros(1, 1, device=dev, dtype=torch.int32)
+    for args, kw in (((table, hidden, 1, 40), {}),                       # two rows, not one
+                     ((table, hidden.repeat(3, 1), 2, 60), {}),          # 40 slots
+                     ((paged, hidden.repeat(2, 1), 1, 80),               # one page of 64
+                      dict(block_table=block_table, n_pages=4, page_size=64)),
+                     ((paged, hidden, 1, 40),                            # five pages
+                      dict(block_table=block_table, n_pages=5, page_size=64))):
+        with pytest.raises(ValueError):
+            prefill_ops.prefill_layers(CFG, *args, eng.inv_freq, **kw)
+    cu = torch.tensor([0, 10, 40], device=dev, dtype=torch.int32)
+    print("[prefill layers] rows of 10 and 30 announced as 20", flush=True)
+    prefill_ops.prefill_layers(CFG, table, hidden, 2, 20, eng.inv_freq, cu=cu)
+    for t in (t for pair in caches for t in pair):
+        used = (t != 0).any(-1).any(1)
+        assert used.sum(1).tolist() == [10, 20] and not bool(used[1, 20:].any())
