@@ -48,7 +48,8 @@ int64_t qf_prefill_layers_workspace(int T, int hidden, int QH, int KVH, int D, i
  * longest row (a token past it in its row is not appended).  Token i of row b
  * goes to slot i of row b: every cache holds S slots at least, which the caller
  * checks; with block_table through it, a page outside the pool writing
- * nothing.  ws: 16-byte aligned, free again when the call's work is done. */
+ * nothing.  ws: 16-byte aligned, of at least the bytes above (else
+ * QF_ERR_SCRATCH_LIMIT), free again when the call's work is done. */
 int qf_prefill_layers(const QfPrefillLayer* layers, int n_layers, void* hidden, int T, int B, int S,
                       const int32_t* cu, const float* inv_freq, const int32_t* block_table,
                       int64_t bt_sb, int pages_per_row, int n_pages, int page_size, void* ws,

@@ -20,11 +20,12 @@
 //
 // Measured on MI355X (kernel trace, 896/4864 widths, 1024 tokens of context),
 // us at B=12 / 32, with the torch projections' kernels at B=12 beside them:
-// QKV + RoPE + append 5.1 / 6.4 (norm 3.6 + GEMM 7.3 + append 4.0), o_proj
-// 4.7 / 4.8 (7.3 + add 4.0), gate/up 6.3 / 8.9 (norm 3.6 + GEMM 10 + silu and
-// product 8), down 6.9 / 8.1 (13.4 + add 4.0), lm_head 46 / 52 (54 + argmax 49).
+// QKV + RoPE + append 4.5 / 6.5 (norm 3.6 + GEMM 7.3 + append 4.0), o_proj
+// 4.0 / 5.1 (7.3 + add 4.0), gate/up 6.6 / 9.0 (norm 3.6 + GEMM 10 + silu and
+// product 8), down 6.7 / 8.0 (13.4 + add 4.0), lm_head 47 / 53 (54 + argmax 49).
 // The first four are bound by launch latency and the round trip of their
-// loads (1.6-17 MB of weights at 0.4-2.4 TB/s), the lm_head by HBM (5.9 TB/s).
+// loads (at B=12 1.6-17 MB of weights at 0.4-2.6 TB/s), the lm_head by HBM
+// (5.8 TB/s).
 //
 // Replaces the torch op sequence of _decode_step_static
 // (student_engine.py:896-982); same rounding points as decode_step.hip.
@@ -103,7 +104,8 @@ __device__ __forceinline__ f16x8 wide_operand(const f16* xs, int K, int kb, int 
 // NaN.  A surplus block is a (non-temporal) buffer load past its range, so it
 // costs neither traffic nor selects on its registers (MI355X, a step of 12 rows
 // and 24 layers: 751.6 us against 753.9 with selects, 749.9 with re-read tiles;
-// the attention half at 4 rows 319 against 323 and 322).  rb is wave-uniform; one past nrb reads zeros.
+// the attention half at 4 rows 319 against 323 and 322).  rb is wave-uniform;
+// one past nrb reads zeros.
 template <int kBlk>
 __device__ __forceinline__ void share_tiles(f16x8 (&wa)[kBlk], const f16* w, int nkb, int nrb,
                                             int rb, int kb0, int n, int lane) {

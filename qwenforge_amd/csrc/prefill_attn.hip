@@ -978,7 +978,8 @@ static int prefill_launch(Args a, bool rope, bool append, hipStream_t st) {
   } else if (paged) {
     return QF_ERR_INVALID_ARG;  // paged prefill always appends
   }
-  // One eight-wave workgroup per (query tile, b * QH + q head).
+  // One workgroup per (query tile, b * QH + q head): eight waves, or four with
+  // one wave group.
   if ((int64_t)grid.x * B * QH > 0x7fffffff) return QF_ERR_UNSUPPORTED;
   const dim3 lgrid((unsigned)(grid.x * B * QH));
   // Two wave groups per query tile (four, one 16-wave workgroup per CU, were

@@ -529,8 +529,10 @@ static int launch_as(GemmArgs a, hipStream_t st) {
 //   - 128 x 128, half the operand bytes per product of 64 x 64, from nine
 //     tiles per 16 CUs on for gate/up (152 tiles at 256 tokens: 13.8 against
 //     16.1; 608 at 1024: 28.7 against 40.1) and from thirteen for the others
-//     (down, unsplit, at 4096 tokens, 224 tiles: 58.4 against 65.8; at 2048,
-//     112 tiles: 56.8 against 33.8; QKV at 2048, 144 tiles: 17.6 against 17.7);
+//     (kernel trace, 128 / 64: QKV at 2560 tokens, 180 tiles, 22.2 / 21.8, 3072,
+//     216, 22.1 / 23.4, 4096, 288, 26.2 / 32.5; o_proj at 2048, 112, 18.6 /
+//     12.9, 2560, 140, 19.4 / 17.3, 4096, 224, 19.0 / 22.0 -- and ahead by 2 at
+//     3072 and 3584 already, 168 and 196 tiles, where QKV is not);
 //   - gate/up 160 features wide from two tiles per CU on: its 9728 rows then
 //     fill whole rounds of workgroups (two per CU) at 1024 x n tokens (28.2
 //     against 28.7, at 4096 81.7 against 88.4, at 8192 160 against 199);
@@ -581,9 +583,9 @@ static int shares128(int T, int N, int K, int slots) {
 // stages deep with a CU to itself while that allows two shares, two stages and
 // two workgroups per CU past that.  Measured on MI355X for the whole prefill of
 // 24 layers, us, unsplit or in 64 x 64 shares merged behind a ticket / this
-// rule: 64 tokens 1263 / 1221, 300 1539 / 1495, 512 1792 / 1763; 600 1852 /
-// 1750, 1024 2314 / 2209, 1280 2954 / 2704, 2048 3736 / 3381; 2400 4667 / 4117,
-// 3000 5287 / 4417, 4096 6309 / 5943.  Across the first line: seven 128 x 128
+// rule: 64 tokens 1242 / 1206, 300 1522 / 1496, 512 1771 / 1755; 600 1832 /
+// 1749, 1024 2312 / 2224, 1280 2947 / 2720, 2048 3744 / 3404; 2400 4653 / 4176,
+// 3000 5243 / 4500, 4096 6325 / 6005.  Across the first line: seven 128 x 128
 // shares at 512 tokens 1785, three 64 x 64 ones at 600 1771.
 static KSplit k_split(int T, int N, int K, int cus) {
   const int64_t t64 = (int64_t)((N + 63) / 64) * ((T + 63) / 64);
