@@ -20,12 +20,12 @@
 //
 // Measured on MI355X (kernel trace, 896/4864 widths, 1024 tokens of context),
 // us at B=12 / 32, with the torch projections' kernels at B=12 beside them:
-// QKV + RoPE + append 4.5 / 6.5 (norm 3.6 + GEMM 7.3 + append 4.0), o_proj
-// 4.0 / 5.1 (7.3 + add 4.0), gate/up 6.6 / 9.0 (norm 3.6 + GEMM 10 + silu and
-// product 8), down 6.7 / 8.0 (13.4 + add 4.0), lm_head 47 / 53 (54 + argmax 49).
+// QKV + RoPE + append 4.4 / 6.6 (norm 3.6 + GEMM 7.3 + append 4.0), o_proj
+// 4.1 / 5.2 (7.3 + add 4.0), gate/up 6.4 / 8.9 (norm 3.6 + GEMM 10 + silu and
+// product 8), down 6.9 / 8.1 (13.4 + add 4.0), lm_head 46 / 53 (54 + argmax 49).
 // The first four are bound by launch latency and the round trip of their
-// loads (at B=12 1.6-17 MB of weights at 0.4-2.6 TB/s), the lm_head by HBM
-// (5.8 TB/s).
+// loads (at B=12 1.6-17 MB of weights at 0.4-2.7 TB/s), the lm_head by HBM
+// (5.9 TB/s).
 //
 // Replaces the torch op sequence of _decode_step_static
 // (student_engine.py:896-982); same rounding points as decode_step.hip.
@@ -101,21 +101,21 @@ __device__ __forceinline__ f16x8 wide_operand(const f16* xs, int K, int kb, int 
 
 // The weight tiles of k blocks [kb0, kb0 + n) of row block rb, zeros past n: a
 // real tile re-read there could hold infinities, which zero columns turn into
-// NaN.  A surplus block is a (non-temporal) buffer load past its range, so it
-// costs neither traffic nor selects on its registers (MI355X, a step of 12 rows
-// and 24 layers: 751.6 us against 753.9 with selects, 749.9 with re-read tiles;
-// the attention half at 4 rows 319 against 323 and 322).  rb is wave-uniform;
-// one past nrb reads zeros.
+// NaN.  The buffer ends after this wave's share (all of it wave-uniform), so a
+// surplus block costs neither traffic nor selects (non-temporal like
+// tile_load).  rb past nrb: zeros.  MI355X, us for 24 layers, tiles re-read /
+// an out-of-range offset a surplus block (in the lanes) / this: the MLP half at
+// 4 rows 267 / 271 / 259, the attention half 322 / 319 / 316, a step of 12 rows
+// 750 / 752 / 741, of 32 951 / - / 946.
 template <int kBlk>
 __device__ __forceinline__ void share_tiles(f16x8 (&wa)[kBlk], const f16* w, int nkb, int nrb,
                                             int rb, int kb0, int n, int lane) {
-  const __amdgpu_buffer_rsrc_t r =
-      buffer_rsrc(w + (int64_t)rb * nkb * 512, rb < nrb ? nkb * 1024 : 0);
+  const __amdgpu_buffer_rsrc_t r = buffer_rsrc(w + ((int64_t)rb * nkb + kb0) * 512,
+                                               rb < nrb && n > 0 ? n * 1024 : 0);
 #pragma unroll
   for (int t = 0; t < kBlk; ++t)
     wa[t] = __builtin_bit_cast(
-        f16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                   r, t < n ? ((kb0 + t) * 64 + lane) * 16 : 0x7ffffff0, 0, kNt));
+        f16x8, __builtin_amdgcn_raw_buffer_load_b128(r, t * 1024 + lane * 16, 0, kNt));
 }
 
 // This wave's k blocks [kb0, kb0 + n) of one row block against every column
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kNT) void wide_qkv_kernel(QkvArgs a) {
   constexpr int NC = col_blocks(kRows);
   __shared__ __attribute__((aligned(16))) f16 xs[kNW * kRows * (kMaxNormK + kPad)];
   __shared__ f32x4 part[kNW][NC][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = touch_arg_lines(a.K, a.x, a.bias, a.write_index, a.slots), nkb = K / 32;
   const int per = (nkb + kNW - 1) / kNW, kb0 = w * per, n = min(per, nkb - kb0);
   const int rb = blockIdx.x;
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(kNT) void wide_gate_up_kernel(GateUpArgs a) {
   constexpr int NC = col_blocks(kRows);
   __shared__ __attribute__((aligned(16))) f16 xs[kNW * kRows * (kMaxNormK + kPad)];
   __shared__ f32x4 part[kNW][kRB * NC][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = a.K, nkb = K / 32, nrb = a.I / 8;
   const int per = (nkb + kNW - 1) / kNW, kb0 = w * per, n = min(per, nkb - kb0);
   const int rb0 = blockIdx.x * kRB;
@@ -571,9 +571,9 @@ static bool wide_rows(int B) { return B >= 5 && B <= QF_WIDE_MAX_B; }
   }
 
 // One row per wave up to 4 rows.  Measured on MI355X (weights past the MALL):
-// at B=4 3.47 us against 4.04 for the 1..4-row form this replaced, whose
+// at B=4 3.14 us against 4.04 for the 1..4-row form this replaced, whose
 // workgroup reduced every row together and read its operands with LDS bank
-// conflicts; B=2 3.48.
+// conflicts; B=2 3.13 (3.32 at both before share_tiles).
 void qf::step::launch_qkv_tiles(const QkvArgs& a, bool paged, bool positions, hipStream_t st) {
   const dim3 grid((a.QH + 2 * a.KVH) * 4), block(kNT);
   if (a.B > 4) {  // positions only: the 5..32-row entry point takes no tables
@@ -593,9 +593,10 @@ void qf::step::launch_qkv_tiles(const QkvArgs& a, bool paged, bool positions, hi
 // Three row blocks per workgroup: the 608 of Qwen2.5-0.5B then take 203
 // workgroups, one round of the CUs, and the rows are staged a third as often
 // (MI355X, weights past the MALL, us for 1 / 2 / 3 / 4 blocks: B=12 6.50 /
-// 6.64 / 5.70 / 6.30, B=32 10.5 / 11.5 / 8.4 / 9.1).  Up to 8 rows the two-row
-// instance: at B=4 5.53 against 6.28 with one row per wave, and 6.03 for
-// rms_gate_up_swiglu_mfma_kernel (B=3 5.54 against 5.78).
+// 6.64 / 5.70 / 6.30, B=32 10.5 / 11.5 / 8.4 / 9.1; with share_tiles three take
+// 5.49 and 8.14).  Up to 8 rows the two-row instance: at B=4 5.21, before
+// share_tiles 5.51 against 6.28 with one row per wave and 6.03 for
+// rms_gate_up_swiglu_mfma_kernel (B=3 5.20, 5.51 against 5.78).
 void qf::step::launch_gate_up_tiles(const GateUpArgs& a, hipStream_t st) {
   constexpr int kRB = 3;
   const dim3 grid((a.I / 8 + kRB - 1) / kRB), block(kNT);

@@ -213,8 +213,8 @@ class DecodeEngine:
         shapes whose weights pack into tiles; other batches and shapes keep
         the torch projections.  Measured on MI355X at Qwen2.5-0.5B shape and
         1024 tokens of context, ms per step, torch projections / wide: B=5
-        1.68 / 0.70, B=8 1.73 / 0.72, B=12 1.71 / 0.75, B=16 1.70 / 0.78, B=32
-        1.97 / 0.95."""
+        1.69 / 0.69, B=8 1.73 / 0.71, B=12 1.71 / 0.74, B=16 1.70 / 0.78, B=32
+        1.98 / 0.95."""
         cfg = self.cfg
         if not (self.fused_step and self.tile_weights
                 and wide_ops.MIN_BATCH <= batch <= wide_ops.MAX_BATCH
